@@ -726,6 +726,9 @@ struct AlignParams {
     const uint32_t* order;       // processing order of the batch's anchors, or null
     // seeded alignment: every read's bucket (offset, count) and seed per map, read-major
     const uint2* bucketOf; const uint16_t* seeds; int M; int k; int thr;
+    // anchors (indices within the batch) that the matrix kernel leaves to a scan of every
+    // shift, and their number
+    uint32_t* list; uint32_t* listCount;
 };
 
 struct ShdResult { int score, overlap, shift, nOps, valid; };
@@ -913,23 +916,13 @@ __device__ __forceinline__ int chooseOrientation(const ShdResult& f, const ShdRe
 
 constexpr int kAlignWaves = kBlock / kWave;
 
-__global__ void __launch_bounds__(kBlock)
-k_align(AlignParams p){
-    // per wave: 6 planes (anchor hi/lo, candidate fwd hi/lo, candidate rc hi/lo) stored as
-    // (word i+1, word i) pairs so one 64-bit LDS read feeds a funnel shift
-    __shared__ uint2 planes[kAlignWaves][6][kMaxHiLoWords + 1];
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    // workgroups stride over the pairs, kAlignWaves at a time (the same trip count for the
-    // whole workgroup, which meets the barriers every time)
-    for(uint64_t base = uint64_t(blockIdx.x) * kAlignWaves; base < p.total; base += uint64_t(gridDim.x) * kAlignWaves){
-    const uint32_t c = uint32_t(base) + uint32_t(wave);
-    const bool active = c < p.total;
-    uint32_t id = 0;
-    uint64_t a = 0;
+// Both alignments of pair c (anchor a, candidate id) by one wavefront, whose planes are staged
+// in LDS (per wave 6: anchor hi/lo, candidate fwd hi/lo, candidate rc hi/lo) as (word i+1,
+// word i) pairs so one 64-bit read feeds a funnel shift. The workgroup's waves meet the
+// barrier together (active: this wave has a pair).
+__device__ __forceinline__ void alignPair(const AlignParams& p, uint2 (*planes)[kMaxHiLoWords + 1], bool active, uint64_t a,
+                                          uint32_t id, uint64_t c, int lane){
     if(active){
-        id = p.ids[c];
-        a = p.b0 + p.anchorOf[c];
         const int W = p.W;
         const uint32_t* ah = p.hilo + a * uint64_t(4 * W);
         const uint32_t* ch = p.hilo + uint64_t(id) * uint64_t(4 * W);
@@ -939,34 +932,64 @@ k_align(AlignParams p){
             const int w = q - pl * (W + 1);
             const uint32_t x0 = w < W ? src[pl][w] : 0u;
             const uint32_t x1 = w + 1 < W ? src[pl][w + 1] : 0u;
-            planes[wave][pl][w] = make_uint2(x1, x0);
+            planes[pl][w] = make_uint2(x1, x0);
         }
     }
     __syncthreads();
     if(active){
-    const int La = p.len[a];
-    const int Lc = p.len[id];
-    ShdResult f, r;
-    alignBoth(planes[wave][0], planes[wave][1], planes[wave][2], planes[wave][3], planes[wave][4], planes[wave][5],
-              La, Lc, p, lane, f, r);
-    const int flag = chooseOrientation(f, r, La, p);
-    if(lane == 0){
-        AlignBest b;
-        const ShdResult& s = flag == 2 ? r : f;
-        b.shift = s.shift;
-        b.overlap = s.overlap;
-        b.nOps = s.nOps;
-        b.orientation = flag;
-        p.best[c] = b;
-        if(p.dbg){
-            int* d = p.dbg + uint64_t(c) * 11;
-            d[0] = f.score; d[1] = f.overlap; d[2] = f.shift; d[3] = f.nOps; d[4] = f.valid;
-            d[5] = r.score; d[6] = r.overlap; d[7] = r.shift; d[8] = r.nOps; d[9] = r.valid;
-            d[10] = flag;
+        const int La = p.len[a];
+        const int Lc = p.len[id];
+        ShdResult f, r;
+        alignBoth(planes[0], planes[1], planes[2], planes[3], planes[4], planes[5], La, Lc, p, lane, f, r);
+        const int flag = chooseOrientation(f, r, La, p);
+        if(lane == 0){
+            AlignBest b;
+            const ShdResult& s = flag == 2 ? r : f;
+            b.shift = s.shift;
+            b.overlap = s.overlap;
+            b.nOps = s.nOps;
+            b.orientation = flag;
+            p.best[c] = b;
+            if(p.dbg){
+                int* d = p.dbg + c * 11;
+                d[0] = f.score; d[1] = f.overlap; d[2] = f.shift; d[3] = f.nOps; d[4] = f.valid;
+                d[5] = r.score; d[6] = r.overlap; d[7] = r.shift; d[8] = r.nOps; d[9] = r.valid;
+                d[10] = flag;
+            }
         }
     }
-    }
     __syncthreads();            // the planes are staged again for the next pairs
+}
+
+// Workgroups stride over the pairs, kAlignWaves at a time (the same trip count for the whole
+// workgroup, which meets the barriers every time).
+__global__ void __launch_bounds__(kBlock)
+k_align(AlignParams p){
+    __shared__ uint2 planes[kAlignWaves][6][kMaxHiLoWords + 1];
+    const int wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1);
+    for(uint64_t base = uint64_t(blockIdx.x) * kAlignWaves; base < p.total; base += uint64_t(gridDim.x) * kAlignWaves){
+        const uint32_t c = uint32_t(base) + uint32_t(wave);
+        const bool active = c < p.total;
+        alignPair(p, planes[wave], active, active ? p.b0 + p.anchorOf[c] : 0, active ? p.ids[c] : 0u, c, lane);
+    }
+}
+
+// The pairs of the listed anchors: workgroups stride over the list, one anchor at a time.
+__global__ void __launch_bounds__(kBlock)
+k_align_listed(AlignParams p){
+    __shared__ uint2 planes[kAlignWaves][6][kMaxHiLoWords + 1];
+    const int wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int count = int(*p.listCount);
+    for(int b = blockIdx.x; b < count; b += gridDim.x){
+        const int i = int(p.list[b]);
+        const uint32_t beg = p.offsets[i], end = p.offsets[i + 1];
+        for(uint64_t base = beg; base < end; base += kAlignWaves){
+            const uint64_t c = base + uint64_t(wave);
+            const bool active = c < end;
+            alignPair(p, planes[wave], active, p.b0 + uint64_t(i), active ? p.ids[c] : 0u, c, lane);
+        }
     }
 }
 
@@ -1296,17 +1319,26 @@ __device__ __forceinline__ void alignLanes(const AlignParams& p, uint64_t a, con
     }
 }
 
-// One wavefront per anchor of the batch, its candidates in chunks of 64 lanes.
 template<int WM>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WM <= 5 ? 8 : 1)))
-k_align_lanes(AlignParams p){
-    if(int(blockIdx.x) >= p.B) return;
-    const int i = batchAnchor(p.order, p.B);
+__device__ __forceinline__ void alignAnchor(const AlignParams& p, int i){
     const uint32_t beg = p.offsets[i];
     const int n = int(p.offsets[i + 1] - beg);
     if(n == 0) return;
     alignLanes<WM>(p, p.b0 + i, p.ids + beg, n, p.best + beg, p.dbg ? p.dbg + uint64_t(beg) * 11 : nullptr,
                    threadIdx.x);
+}
+
+// One wavefront per anchor of the batch (a grid of p.B), its candidates in chunks of 64
+// lanes; LISTED: wavefronts striding over the listed anchors.
+template<int WM, bool LISTED>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WM <= 5 ? 8 : 1)))
+k_align_lanes(AlignParams p){
+    if constexpr(LISTED){
+        const int count = int(*p.listCount);
+        for(int b = blockIdx.x; b < count; b += gridDim.x) alignAnchor<WM>(p, int(p.list[b]));
+    }else{
+        if(int(blockIdx.x) < p.B) alignAnchor<WM>(p, batchAnchor(p.order, p.B));
+    }
 }
 
 // Seeded alignment (an addition; the reference has no counterpart): one shift per
@@ -1418,6 +1450,8 @@ k_align_seeded(AlignParams p){
         p.best[beg + c] = b;
     }
 }
+
+#include "align_matrix.hpp"
 
 // Words per plane handled by the lane kernel for reads of W words (0: too long).
 int alignLaneWords(int W){
@@ -3368,7 +3402,7 @@ struct care_ctx {
     // batch working memory
     DBuf raw, uniq, offsets, ids, anchorOf, best, dbg, paired;
     DBuf kId, kShift, kLen, kNops, kOvl, kW, kOrient, kPaired;
-    DBuf slots, recBytes, recOff, recOff64, outBuf, info, msaDbg, counters, scanTmp, scratch, candOver;
+    DBuf slots, recBytes, recOff, recOff64, outBuf, info, msaDbg, counters, scanTmp, scratch, candOver, alignOver;
     // learned seam: classifier (bfloat16 weights then float biases) and feature output
     DBuf seam, featBuf, metaBuf;
     // pinned host words: record bytes (u64) and the error flag (i32) of the last pass
@@ -3667,6 +3701,7 @@ void fillAlignCommon(const care_ctx* ctx, AlignParams& ap){
     ap.maxLen = ctx->maxLen;
     ap.eExact = errorBoundAsInteger(ap.maxErrorRate, ctx->maxLen, ap.eMul, ap.ePre) ? 1 : 0;
     if(!ap.eExact){ ap.eMul = 0; ap.ePre = 0; }
+    ap.list = nullptr; ap.listCount = nullptr;
     ap.order = nullptr;
     ap.bucketOf = ctx->bucketOf.as<uint2>(); ap.seeds = ctx->seeds.as<uint16_t>();
     ap.M = ctx->M; ap.k = ctx->k; ap.thr = ctx->thr;
@@ -3963,8 +3998,44 @@ int batchOrder(care_ctx* ctx, uint64_t b0, int B, const uint32_t** out){
     return CARE_OK;
 }
 
-// The alignment kernel of a staged batch: the seeded kernel (seeded alignment), the
-// lane-per-candidate kernel (wm > 0), or the wavefront-per-pair kernel over `total` pairs.
+// Whether a staged batch aligns with the matrix kernel: the default variant, while the error
+// rate leaves the filter its selectivity (at 0.3 it takes 0.43 ms where the lane scan takes
+// 1.14 ms on 80,000 reads of 150 bases; beyond, an overlap of 45 bases passes by chance in
+// over 0.1% of the shifts) and while a read has at least kMatrixMinShifts shifts to scan per
+// direction: blocks cost the same for one shift as for 32 (reads of 40 bases: 0.39 ms
+// against 0.39 ms of the lane scan, of 36: 0.40 against 0.33, of 44: 0.38 against 0.44).
+bool matrixAlign(const care_ctx* ctx){
+    const int mo = std::max(ctx->o.min_overlap, int(float(ctx->maxLen) * ctx->o.min_overlap_ratio));
+    return !ctx->o.seeded_alignment && ctx->o.align_variant != 1 && ctx->W <= kMaxHiLoWords &&
+           ctx->maxLen - mo >= kMatrixMinShifts &&
+           ctx->o.max_error_rate >= 0.0f && ctx->o.max_error_rate <= kMatrixMaxRate;
+}
+
+// The list of anchors the matrix kernel leaves to a scan, for batches of at most B.
+hipError_t prepareAlignList(care_ctx* ctx, int B, AlignParams& ap){
+    if(!matrixAlign(ctx)) return hipSuccess;
+    const hipError_t e = ctx->alignOver.ensure(size_t(B) * 4 + 16);
+    if(e != hipSuccess) return e;
+    ap.listCount = ctx->alignOver.as<uint32_t>();
+    ap.list = ctx->alignOver.as<uint32_t>() + 4;
+    return hipSuccess;
+}
+
+template<bool LISTED>
+hipError_t launchAlignLanes(const AlignParams& ap, int grid, int wm, hipStream_t st){
+    switch(wm){
+        case 2: k_align_lanes<2, LISTED><<<grid, kWave, 0, st>>>(ap); break;
+        case 4: k_align_lanes<4, LISTED><<<grid, kWave, 0, st>>>(ap); break;
+        case 5: k_align_lanes<5, LISTED><<<grid, kWave, 0, st>>>(ap); break;
+        case 8: k_align_lanes<8, LISTED><<<grid, kWave, 0, st>>>(ap); break;
+        default: k_align_lanes<11, LISTED><<<grid, kWave, 0, st>>>(ap); break;
+    }
+    return hipGetLastError();
+}
+
+// The alignment kernel of a staged batch: the seeded kernel (seeded alignment), the matrix
+// kernel followed by the scan of the anchors it listed, the lane-per-candidate kernel
+// (wm > 0), or the wavefront-per-pair kernel over `total` pairs.
 hipError_t launchAlign(const care_ctx* ctx, const AlignParams& ap, int B, uint32_t total, int wm, hipStream_t st){
     if(ctx->o.seeded_alignment){
         switch(alignLaneWords(ctx->W)){
@@ -3975,16 +4046,29 @@ hipError_t launchAlign(const care_ctx* ctx, const AlignParams& ap, int B, uint32
             case 11: k_align_seeded<11><<<B, kWave, 0, st>>>(ap); break;
             default: return hipErrorInvalidValue;      // rejected before any batch runs
         }
-    }else{
-        switch(wm){
-            case 2: k_align_lanes<2><<<B, kWave, 0, st>>>(ap); break;
-            case 4: k_align_lanes<4><<<B, kWave, 0, st>>>(ap); break;
-            case 5: k_align_lanes<5><<<B, kWave, 0, st>>>(ap); break;
-            case 8: k_align_lanes<8><<<B, kWave, 0, st>>>(ap); break;
-            case 11: k_align_lanes<11><<<B, kWave, 0, st>>>(ap); break;
-            default: k_align<<<gridFor(uint64_t(total) * kWave, kBlock), kBlock, 0, st>>>(ap); break;
-        }
+        return hipGetLastError();
     }
+    if(matrixAlign(ctx)){
+        k_zero_u32<<<1, 64, 0, st>>>(ap.listCount, 1);
+        const size_t lds = size_t(matrixLds(ctx->W).bytes);
+        switch((ctx->W + 1) / 2){
+            case 0: case 1: k_align_matrix<1><<<B, kWave, lds, st>>>(ap); break;
+            case 2: k_align_matrix<2><<<B, kWave, lds, st>>>(ap); break;
+            case 3: k_align_matrix<3><<<B, kWave, lds, st>>>(ap); break;
+            case 4: k_align_matrix<4><<<B, kWave, lds, st>>>(ap); break;
+            case 5: case 6: k_align_matrix<6><<<B, kWave, lds, st>>>(ap); break;
+            case 7: case 8: k_align_matrix<8><<<B, kWave, lds, st>>>(ap); break;
+            case 9: case 10: case 11: case 12: k_align_matrix<12><<<B, kWave, lds, st>>>(ap); break;
+            default: k_align_matrix<16><<<B, kWave, lds, st>>>(ap); break;
+        }
+        const hipError_t e = hipGetLastError();
+        if(e != hipSuccess) return e;
+        if(alignLaneWords(ctx->W) > 0) return launchAlignLanes<true>(ap, std::min(B, 8192), alignLaneWords(ctx->W), st);
+        k_align_listed<<<std::min(B, 8192), kBlock, 0, st>>>(ap);
+        return hipGetLastError();
+    }
+    if(wm > 0) return launchAlignLanes<false>(ap, B, wm, st);
+    k_align<<<gridFor(uint64_t(total) * kWave, kBlock), kBlock, 0, st>>>(ap);
     return hipGetLastError();
 }
 
@@ -4105,7 +4189,7 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     if(ctx->o.keep_intermediates) HIPCHECK(ctx->dbg.ensure(T * 11 * sizeof(int)));
     // anchorOf is read by the wavefront-per-pair alignment and by candidate correction
     const int wm = ctx->o.align_variant == 1 ? 0 : alignLaneWords(ctx->W);
-    const bool needAnchorOf = wm == 0 || ctx->o.correct_candidates != 0;
+    const bool needAnchorOf = (wm == 0 && !matrixAlign(ctx)) || ctx->o.correct_candidates != 0;
     k_compact<<<(B + kBlock / kWave - 1) / (kBlock / kWave), kBlock, 0, st>>>(
         ctx->raw.as<uint32_t>(), capPerAnchor, ctx->offsets.as<uint32_t>(), B, ctx->ids.as<uint32_t>(),
         needAnchorOf ? ctx->anchorOf.as<uint32_t>() : nullptr);
@@ -4124,6 +4208,7 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     ap.best = ctx->best.as<AlignBest>(); ap.dbg = ctx->o.keep_intermediates ? ctx->dbg.as<int>() : nullptr;
     ap.offsets = ctx->offsets.as<uint32_t>(); ap.B = B; ap.maxLen = ctx->maxLen;
     ap.order = order;
+    HIPCHECK(prepareAlignList(ctx, B, ap));
     if(total) HIPCHECK(launchAlign(ctx, ap, B, total, wm, st));
     HIPCHECK(hipEventRecord(ctx->ev[2], st));
 
@@ -4369,6 +4454,7 @@ int prepareStaged(care_ctx* ctx, int Bmax, uint64_t cap, StagedLaunch& L){
     ap.ids = ctx->ids.as<uint32_t>(); ap.anchorOf = nullptr; ap.total = 0;
     ap.best = ctx->best.as<AlignBest>(); ap.dbg = nullptr;
     ap.offsets = ctx->offsets.as<uint32_t>(); ap.maxLen = ctx->maxLen;
+    HIPCHECK(prepareAlignList(ctx, Bmax, ap));
 
     MsaParams& mp = L.mp;
     fillMsaCommon(ctx, mp);
@@ -4659,7 +4745,7 @@ void care_hip_destroy(care_ctx* ctx){
                    &ctx->fqHdrLen, &ctx->fqSeq, &ctx->fqQual, &ctx->mRec, &ctx->mOff, &ctx->mKeyIn, &ctx->mKeyOut,
                    &ctx->mIdxIn, &ctx->mIdxOut, &ctx->mRunBeg, &ctx->mRunEnd, &ctx->mPlan, &ctx->mSize, &ctx->mOutOff,
                    &ctx->mText, &ctx->mErr, &ctx->candSlots, &ctx->candBytes, &ctx->insSize, &ctx->insOff,
-                   &ctx->insSrc, &ctx->hqAnchor, &ctx->seeds, &ctx->pipeOut[0], &ctx->pipeOut[1]}){
+                   &ctx->insSrc, &ctx->hqAnchor, &ctx->seeds, &ctx->alignOver, &ctx->pipeOut[0], &ctx->pipeOut[1]}){
         b->release();
     }
     if(ctx->fusedExec) (void)hipGraphExecDestroy(ctx->fusedExec);
@@ -6278,7 +6364,8 @@ static int care_hip_correct_body(care_ctx* ctx, uint64_t first, uint64_t n, size
     // correction with the lane-per-candidate or seeded alignment; candidate correction,
     // intermediate dumps and feature output synchronize per batch
     const bool pipelined = !fused && !cands && !ctx->o.keep_intermediates && !ctx->featActive && !ctx->o.sync_batches &&
-                           (ctx->o.seeded_alignment || (ctx->o.align_variant != 1 && alignLaneWords(ctx->W) > 0));
+                           (ctx->o.seeded_alignment || matrixAlign(ctx) ||
+                            (ctx->o.align_variant != 1 && alignLaneWords(ctx->W) > 0));
     unsigned long long pipeGathered = 0;
     const auto t0 = std::chrono::steady_clock::now();
     if(fused){
