@@ -296,6 +296,31 @@ __global__ void k_repack_rows(const uint8_t* __restrict__ src, size_t sp, uint8_
     }
 }
 
+// Per read its length and, in the upper 16 bits, the least quality weight of its bases in
+// units of 2^-16, rounded down (1 without qualities). Read by the high-quality test of the
+// MSA stage, which gathers it in place of the length.
+__global__ void __launch_bounds__(256) k_len_weight(const int* __restrict__ len, const uint8_t* __restrict__ qual, size_t qdpitch,
+                                                    const float* __restrict__ qweight, uint64_t n, uint32_t* __restrict__ out){
+    FOR_GRID(r, n){
+        const int L = len[r];
+        float w = 1.0f;
+        if(qual){
+            const uint4* row = reinterpret_cast<const uint4*>(qual + qdpitch * r);
+            uint32_t least = 255;
+            for(int c = 0; 16 * c < L; c++){
+                const uint4 v = row[c];
+                const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+                #pragma unroll
+                for(int i = 0; i < 16; i++){
+                    if(16 * c + i < L) least = min(least, (x[i >> 2] >> (8 * (i & 3))) & 0xFFu);
+                }
+            }
+            w = qweight[least];         // the weights do not fall as the quality rises
+        }
+        out[r] = uint32_t(L) | (min(uint32_t(w * 65536.0f), 65535u) << 16);
+    }
+}
+
 __global__ void k_iota(uint32_t* v, uint64_t n){
     FOR_GRID(i, n) v[i] = uint32_t(i);
 }
@@ -1468,6 +1493,7 @@ int alignLaneWords(int W){
 struct MsaParams {
     const uint32_t* enc; size_t pitch; const int* len; const uint8_t* qual; size_t qpitch; const uint8_t* ambig;
     size_t qdpitch;                 // device quality row pitch (qpitch rounded up to 16 bytes)
+    const uint32_t* lenWeight;      // per read: length | least quality weight of its bases << 16 (k_len_weight)
     int varLen;                     // reads of different lengths: stage only what each candidate covers
     const float* qweight;
     uint64_t b0;
@@ -1550,12 +1576,20 @@ struct MsaTile {
 // one 16-byte store per chunk.
 __host__ __device__ inline int qStride(int maxLen){ return (maxLen + 15) & ~15; }
 
+// LDS of the high-quality test of certainHighQuality: four arrays over the anchor's columns and
+// the anchor's 2-bit row between zero words.
+__host__ __device__ inline int certainColumns(int maxLen){ return ((maxLen + 63) & ~63) + 64; }
+__host__ __device__ inline size_t certainLdsBytes(int maxLen){
+    return 4 * (4 * size_t(certainColumns(maxLen)) + size_t((maxLen + 15) >> 4) + 4);
+}
+
 // Bytes of the one-wavefront MSA's tile region: the candidate tile, which the learned seam
 // (kSeamLdsBytes) and the consensus of candidate correction (maxCols bytes) reuse.
 __host__ __device__ inline size_t waveTileRegion(int T, int W, int maxLen, bool useQ, bool seam, int maxCols){
     size_t b = size_t(T) * (20 + 8 * size_t(W)) + (useQ ? size_t(T) * size_t(qStride(maxLen)) : 0);
     if(seam && b < kSeamLdsBytes) b = kSeamLdsBytes;
     if(b < size_t(maxCols)) b = size_t(maxCols);
+    b = std::max(b, certainLdsBytes(maxLen));
     return (b + 15) / 16 * 16;
 }
 
@@ -2492,6 +2526,196 @@ __device__ __forceinline__ void emitCandidateRecords(const MsaParams& p, const A
     }
 }
 
+// Whether the anchor is certain to be corrected as a high-quality anchor, and with which edits:
+// decided from bounds, so that most anchors of an ordinary read set end here, before any
+// quality or candidate row is staged. k_msa_wave went 6.8 -> 2.2 ms on 1.0M reads of 150
+// bases (87% end here without a record, against 0.2% whose MSA is built for none), 16.0 ->
+// 10.3 ms on 1.03M reads of 100..250 bases with repeats, 2.1 -> 1.5 ms on 594,000 reads of 101
+// bases with 1% errors and no qualities; what is left there are repeat copies and refinements.
+//
+// In an anchor column where every candidate agrees with the anchor the consensus is the
+// anchor's base and the support is exactly 1 (the other bases' weights are +0). In the other
+// columns coverage and base counts are exact, and weights are bounded: a candidate weighs w
+// times its quality weight, at least w times the least of its read and at most w. With S a
+// lower bound of all weights of the column and D an upper bound of the disagreeing ones, the
+// consensus is the anchor's base with a support of at least 1 - D / S where that is over one
+// half; with B a lower bound of the weights of one other base and R an upper bound of all
+// the rest (at most 1 each), it is that base with at least B / (B + R) where B > R. When
+// every column is decided, no refinement applies (no edit, or no base other than a column's
+// consensus reaches the count that starts one), and the bounds meet the thresholds of the
+// decision below by kCertainMargin (far above what rounding moves the reference's float
+// sums), the anchor is high quality and its edits are the decided columns that differ. Otherwise
+// nothing is known and the MSA is built. Sums are integers in units of 2^-12 (lower bounds
+// rounded down, upper ones up).
+//
+// S comes from a difference array over the columns (three LDS adds per candidate, then a
+// wave scan; the column's coverage in the upper 10 bits), the rest from the mismatch positions
+// of the candidates that have any. A reverse-complement candidate's qualities are those of
+// its read only for positions from qpitch - len on (below, the row holds what follows the
+// read).
+//
+// get(j, c) fills candidate j of cnt (lanes take j = lane, lane + 64, ...) and returns whether
+// it is kept. Edits: one bit and the corrected base (2 bits) per slot (column lane + 64 k).
+struct CertainCand { uint32_t id; int shift, len, orient, nOps; float w, qmin; };
+constexpr float kCertainMargin = 1e-3f;
+constexpr int kCertainMaxCands = 960;       // coverage and weight fields hold this many
+
+template<int KC, int QM, class Get>
+__device__ __forceinline__ bool certainHighQuality(const MsaParams& p, uint64_t a, int La, const uint32_t* arow,
+                                                   uint32_t* work, int lane, int cnt, uint32_t& editBits,
+                                                   uint32_t& corrBases, int& nEdits, Get&& get){
+    // (a support above one half makes the anchor's base the consensus)
+    const float tMin = fmaxf(fmaxf(p.minThr, p.hqMinT), 0.5f) + kCertainMargin;
+    const float tAvg = fmaxf(p.avgThr, p.hqAvgT) + kCertainMargin;
+    const int cols = certainColumns(p.maxLen);
+    uint32_t* const diff = work;
+    uint32_t* const dis = work + cols;              // upper bound of the disagreeing weights
+    uint32_t* const low = dis + cols;               // their lower bound
+    uint32_t* const alt = low + cols;               // counts by base xor the anchor's (1..3), 10 bits each
+    uint32_t* const aw = alt + cols + 1;            // aw[-1..RW] around the anchor's row
+    const int RW = tileRowWords(p.maxLen);
+    for(int q = lane; q < 4 * cols; q += kWave) work[q] = 0;
+    for(int q = lane; q < RW + 2; q += kWave) aw[q - 1] = q >= 1 && q <= RW ? arow[q - 1] : 0u;
+    __syncthreads();
+    int ops = 0;
+    for(int base = 0; base < cnt; base += kWave){
+        CertainCand c;
+        const bool kept = get(base + lane, c);
+        if(kept){
+            ops += c.nOps;
+            const int cb = max(c.shift, 0), ce = min(c.shift + c.len, La);
+            const bool rc = c.orient != 1;
+            const int qfrom = QM == 1 && rc ? int(p.qpitch) - c.len : 0;    // first position with a quality of the read
+            const int wb = max(c.shift + qfrom, 0);
+            const uint32_t wlow = uint32_t(fmaxf(c.w * c.qmin, 0.0f) * 4096.0f);
+            const uint32_t wf = wb < ce ? wlow : 0u;
+            atomicAdd(&diff[cb], 1u << 22);
+            if(wf) atomicAdd(&diff[wb], wf);
+            atomicAdd(&diff[ce], 0u - (1u << 22) - wf);
+            // positions where it differs from the anchor (16 bases per word)
+            if(c.nOps > 0 && c.nOps <= La){
+                const uint32_t df = uint32_t(c.w * 4096.0f) + 1u;
+                const uint32_t* crow = rc ? p.rcenc + uint64_t(c.id) * uint64_t(2 * p.W) : p.enc + p.pitch * c.id;
+                const int cbeg = max(-c.shift, 0), cend = min(c.len, La - c.shift);
+                int left = c.nOps;
+                for(int k = cbeg >> 4; 16 * k < cend && left > 0; k++){
+                    const int o = 16 * k + c.shift;             // anchor position of the word's first base, > -16
+                    const uint32_t w0 = aw[o >> 4], w1 = aw[(o >> 4) + 1];
+                    const uint32_t av = uint32_t((((uint64_t(w0) << 32) | w1) << (2 * (o & 15))) >> 32);
+                    const uint32_t diffBits = crow[k] ^ av;
+                    uint32_t x = (diffBits | (diffBits >> 1)) & 0x55555555u;
+                    const int lo = max(cbeg - 16 * k, 0), hi = min(cend - 16 * k, 16);
+                    x &= (0xFFFFFFFFu >> (2 * lo)) & uint32_t(~(0xFFFFFFFFull >> (2 * hi)));
+                    while(x){
+                        const int pos = __clz(int(x)) >> 1;
+                        x &= ~(0xC0000000u >> (2 * pos));
+                        const int code = int(diffBits >> (30 - 2 * pos)) & 3;       // 1..3
+                        atomicAdd(&dis[o + pos], df);
+                        atomicAdd(&alt[o + pos], 1u << (10 * (code - 1)));
+                        if(16 * k + pos >= qfrom) atomicAdd(&low[o + pos], wlow);
+                        left--;
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if(waveReduce(ops, OpSum(), 0) > La) return false;
+    // the anchor's own weight in every column
+    const float qa = QM == 1 ? float(p.lenWeight[a] >> 16) * (1.0f / 65536.0f) : 1.0f;
+    const uint32_t own = uint32_t(qa * 4096.0f);
+    uint32_t carry = 0;
+    int mincov = INT_MAX, rival = 0;
+    float worst = 0.0f, defect = 0.0f;
+    bool decided = true;
+    editBits = 0;
+    corrBases = 0;
+    nEdits = 0;
+    #pragma unroll
+    for(int k = 0; k < KC; k++){
+        if(64 * k >= La) break;
+        const int c = lane + kWave * k;
+        const uint32_t v = uint32_t(waveInclusiveSum(int(diff[c]))) + carry;
+        carry = uint32_t(__builtin_amdgcn_readlane(int(v), 63));
+        bool edit = false;
+        if(c < La){
+            const int cov = int(v >> 22) + 1;
+            mincov = min(mincov, cov);
+            const uint32_t counts = alt[c];
+            if(counts){
+                const int n1 = int(counts & 1023u), n2 = int((counts >> 10) & 1023u), n3 = int(counts >> 20);
+                const int best = max(max(n1, n2), n3);
+                const int others = n1 + n2 + n3 - best, agree = cov - best - others;
+                const float d = float(dis[c]), s = float((v & 0x3FFFFFu) + own);
+                float def = d / fmaxf(s, 1.0f);             // 1 - support, at most
+                if(def < 0.5f - kCertainMargin){
+                    rival = max(rival, best);
+                }else{
+                    const int code = n1 == best ? 1 : (n2 == best ? 2 : 3);
+                    const float b = float(low[c]) * (1.0f / 4096.0f) - float(others), r = float(agree + others);
+                    def = r / fmaxf(b + r, 1e-6f);
+                    edit = b > r + kCertainMargin;
+                    decided &= edit;
+                    rival = max(rival, max(agree, others));
+                    editBits |= uint32_t(edit) << k;
+                    const int ab = int((aw[c >> 4] >> (30 - 2 * (c & 15))) & 3u);
+                    corrBases |= uint32_t(ab ^ code) << (2 * k);
+                }
+                worst = fmaxf(worst, def);
+                defect += def;
+            }
+        }
+        nEdits += __popcll(__ballot(edit));
+    }
+    if(__ballot(!decided || !(1.0f - worst >= tMin)) != 0) return false;
+    // with an edit, a base other than the consensus that reaches the threshold starts a refinement
+    if(nEdits > 0 && (nEdits > La / 7 || __ballot(rival >= p.sigThr) != 0)) return false;
+    mincov = waveReduce(mincov, OpMin(), INT_MAX);
+    const int total = waveReduce(int(defect * 65536.0f) + 1, OpSum(), 0);
+    return fgeq(float(mincov), p.minCovThr) && 1.0f - float(total) * (1.0f / 65536.0f) / float(La) >= tAvg;
+}
+
+// Record of a corrected anchor (include/corrector.hpp:1639-1761,
+// include/correctedsequence.hpp:299-387): slots hold the corrected bases (2 bits each), edit
+// bits and whether the slot is an anchor column.
+template<int KC>
+__device__ __forceinline__ void writeRecord(const MsaParams& p, uint64_t a, int i, int La, bool isHQ, bool useEdits, int nEdits,
+                                            uint32_t corrBases, uint32_t editBits, uint32_t isAnchor, int off, int lane,
+                                            int* info){
+    const uint64_t below = lanesBelow(lane);
+    const uint32_t payload = useEdits ? uint32_t(4 + 5 * nEdits) : uint32_t(4 + La);
+    uint8_t* rec = p.slots + size_t(i) * p.slotBytes;
+    if(lane == 0){
+        const uint32_t rid = uint32_t(a);
+        const uint32_t flags = (uint32_t(isHQ) << 31) | (uint32_t(useEdits) << 30) | payload;
+        memcpy(rec, &rid, 4);
+        memcpy(rec + 4, &flags, 4);
+        const int first = useEdits ? nEdits : La;
+        memcpy(rec + 8, &first, 4);
+        p.recBytes[i] = 8 + payload;
+        if(info) info[11] = int(8 + payload);
+    }
+    int running = 0;
+    #pragma unroll
+    for(int k = 0; k < KC; k++){
+        const bool anc = (isAnchor >> k) & 1u;
+        const int q = lane + kWave * k - off;
+        const int cb = int((corrBases >> (2 * k)) & 3u);
+        if(useEdits){
+            const bool e = (editBits >> k) & 1u;
+            const uint64_t mask = __ballot(e);
+            if(e){
+                const int r = running + __popcll(mask & below);
+                memcpy(rec + 12 + 4 * r, &q, 4);
+                rec[12 + 4 * nEdits + r] = uint8_t("ACGT"[cb]);
+            }
+            running += __popcll(mask);
+        }else if(anc){
+            rec[12 + q] = uint8_t("ACGT"[cb]);
+        }
+    }
+}
+
 // Filters, MSA, refinement, decision and record of anchor `a` by one wavefront
 // (include/corrector.hpp:982-1446,1639-1761; src/msa.cpp:9-453,532-734). Its candidates
 // are lst.ids/lst.best/lst.paired[beg, beg+n0); the record goes to slot `i`.
@@ -2541,14 +2765,31 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
         n2 = __popcll(mask);
         uint32_t id = 0;
         int L = 0;
-        float w = 0.0f;
+        float w = 0.0f, qmin = 1.0f;
+        const int no = b.nOps, ov = b.overlap;
         if(keep){
-            const int d = beg + __popcll(mask & below);
             id = lst.ids[beg + lane];
-            L = p.len[id];
-            const int no = b.nOps, ov = b.overlap;
+            const uint32_t lw = p.lenWeight[id];
+            L = int(lw & 0xFFFFu);
+            qmin = float(lw >> 16) * (1.0f / 65536.0f);
             // overlap weight (include/hostdevicefunctions.cuh:93-97)
             w = 1.0f - sqrtf(no / (ov * p.maxErrorRate));
+        }
+        if constexpr(AO && QM != 2){
+            uint32_t editBits, corrBases;
+            int nEdits;
+            if(n2 > 0 && !p.ambig[a] &&
+               certainHighQuality<KC, QM>(p, a, La, arow, reinterpret_cast<uint32_t*>(tile.shift), lane, kWave, editBits,
+                                          corrBases, nEdits, [&](int, CertainCand& c){
+                                              c = CertainCand{id, b.shift, L, b.orientation, no, w, qmin};
+                                              return keep;
+                                          })){
+                if(nEdits > 0) writeRecord<KC>(p, a, i, La, true, true, nEdits, corrBases, editBits, 0u, 0, lane, nullptr);
+                return;
+            }
+        }
+        if(keep){
+            const int d = beg + __popcll(mask & below);
             lst.kId[d] = id; lst.kShift[d] = b.shift; lst.kLen[d] = L; lst.kNops[d] = no; lst.kOvl[d] = ov;
             lst.kOrient[d] = uint8_t(b.orientation); lst.kPaired[d] = pr;
             lst.kW[d] = w;
@@ -2621,9 +2862,34 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
             }
             n2 += __popcll(mask);
         }
+        if constexpr(AO && QM != 2){
+            uint32_t editBits, corrBases;
+            int nEdits;
+            if(n2 > 0 && n2 <= kCertainMaxCands && !p.ambig[a] &&
+               certainHighQuality<KC, QM>(p, a, La, arow, reinterpret_cast<uint32_t*>(tile.shift), lane, n2, editBits,
+                                          corrBases, nEdits, [&](int j, CertainCand& c){
+                                              if(j >= n2) return false;
+                                              c.id = lst.kId[beg + j];
+                                              c.shift = lst.kShift[beg + j];
+                                              c.len = lst.kLen[beg + j];
+                                              c.orient = lst.kOrient[beg + j];
+                                              c.nOps = lst.kNops[beg + j];
+                                              c.w = lst.kW[beg + j];
+                                              c.qmin = QM == 1 ? float(p.lenWeight[c.id] >> 16) * (1.0f / 65536.0f) : 1.0f;
+                                              return true;
+                                          })){
+                if(nEdits > 0) writeRecord<KC>(p, a, i, La, true, true, nEdits, corrBases, editBits, 0u, 0, lane, nullptr);
+                return;
+            }
+        }
     }
     if(info && lane == 0) info[0] = n2;
     if(n2 == 0) return;
+    if constexpr(QM == 1){
+        // the quality-weight table, only for anchors whose MSA is built
+        for(int q = lane; q < 256; q += kWave) const_cast<float*>(tile.qw)[q] = p.qweight[q];
+        __syncthreads();
+    }
 
     // 3) MSA and refinement (include/corrector.hpp:1307-1421; src/msa.cpp:532-734)
     WaveMsa<KC> m;
@@ -2893,37 +3159,7 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
     const bool ambiguous = p.ambig[a] != 0;
     const bool useEdits = !ambiguous && nEdits <= La / 7;
     if(isHQ && useEdits && nEdits == 0) return;
-    const uint32_t payload = useEdits ? uint32_t(4 + 5 * nEdits) : uint32_t(4 + La);
-    uint8_t* rec = p.slots + size_t(i) * p.slotBytes;
-    if(lane == 0){
-        const uint32_t rid = uint32_t(a);
-        const uint32_t flags = (uint32_t(isHQ) << 31) | (uint32_t(useEdits) << 30) | payload;
-        memcpy(rec, &rid, 4);
-        memcpy(rec + 4, &flags, 4);
-        const int first = useEdits ? nEdits : La;
-        memcpy(rec + 8, &first, 4);
-        p.recBytes[i] = 8 + payload;
-        if(info) info[11] = int(8 + payload);
-    }
-    int running = 0;
-    #pragma unroll
-    for(int k = 0; k < KC; k++){
-        const bool anc = (m.isAnchor >> k) & 1u;
-        const int q = lane + kWave * k - off;
-        const int cb = int((corrBases >> (2 * k)) & 3u);
-        if(useEdits){
-            const bool e = (editBits >> k) & 1u;
-            const uint64_t mask = __ballot(e);
-            if(e){
-                const int r = running + __popcll(mask & below);
-                memcpy(rec + 12 + 4 * r, &q, 4);
-                rec[12 + 4 * nEdits + r] = uint8_t("ACGT"[cb]);
-            }
-            running += __popcll(mask);
-        }else if(anc){
-            rec[12 + q] = uint8_t("ACGT"[cb]);
-        }
-    }
+    writeRecord<KC>(p, a, i, La, isHQ, useEdits, nEdits, corrBases, editBits, m.isAnchor, off, lane, info);
 }
 
 template<int KC, bool AO, int QM>
@@ -2936,8 +3172,10 @@ k_msa_wave(MsaParams p){
     MsaTile tile;
     float* sSup;
     carveWaveTile(p, smem, sQw, tile, sSup);
-    if(p.useQ) for(int q = lane; q < 256; q += kWave) sQw[q] = p.qweight[q];
-    __syncthreads();
+    if(QM == 2 && p.useQ){
+        for(int q = lane; q < 256; q += kWave) sQw[q] = p.qweight[q];
+        __syncthreads();
+    }
     const int i = batchAnchor(p.order, p.B);
     const int beg = int(p.offsets[i]);
     const int n0 = int(p.offsets[i + 1]) - beg;
@@ -3402,7 +3640,7 @@ struct care_ctx {
     // batch working memory
     DBuf raw, uniq, offsets, ids, anchorOf, best, dbg, paired;
     DBuf kId, kShift, kLen, kNops, kOvl, kW, kOrient, kPaired;
-    DBuf slots, recBytes, recOff, recOff64, outBuf, info, msaDbg, counters, scanTmp, scratch, candOver, alignOver;
+    DBuf slots, recBytes, recOff, recOff64, outBuf, info, msaDbg, counters, scanTmp, scratch, candOver, alignOver, lenWeight;
     // learned seam: classifier (bfloat16 weights then float biases) and feature output
     DBuf seam, featBuf, metaBuf;
     // pinned host words: record bytes (u64) and the error flag (i32) of the last pass
@@ -3618,6 +3856,7 @@ void fillMsaCommon(const care_ctx* ctx, MsaParams& mp){
     mp.enc = ctx->enc.as<uint32_t>(); mp.pitch = ctx->pitch; mp.len = ctx->len.as<int>();
     mp.qual = ctx->qual.as<uint8_t>(); mp.qpitch = ctx->qpitch; mp.ambig = ctx->ambig.as<uint8_t>();
     mp.qdpitch = ctx->qdpitch;
+    mp.lenWeight = ctx->lenWeight.as<uint32_t>();
     mp.varLen = ctx->varLen ? 1 : 0;
     mp.qweight = ctx->qw.as<float>();
     mp.isPaired = ctx->o.paired; mp.useQ = ctx->o.use_quality_scores;
@@ -4745,7 +4984,7 @@ void care_hip_destroy(care_ctx* ctx){
                    &ctx->fqHdrLen, &ctx->fqSeq, &ctx->fqQual, &ctx->mRec, &ctx->mOff, &ctx->mKeyIn, &ctx->mKeyOut,
                    &ctx->mIdxIn, &ctx->mIdxOut, &ctx->mRunBeg, &ctx->mRunEnd, &ctx->mPlan, &ctx->mSize, &ctx->mOutOff,
                    &ctx->mText, &ctx->mErr, &ctx->candSlots, &ctx->candBytes, &ctx->insSize, &ctx->insOff,
-                   &ctx->insSrc, &ctx->hqAnchor, &ctx->seeds, &ctx->alignOver, &ctx->pipeOut[0], &ctx->pipeOut[1]}){
+                   &ctx->insSrc, &ctx->hqAnchor, &ctx->seeds, &ctx->alignOver, &ctx->lenWeight, &ctx->pipeOut[0], &ctx->pipeOut[1]}){
         b->release();
     }
     if(ctx->fusedExec) (void)hipGraphExecDestroy(ctx->fusedExec);
@@ -4988,6 +5227,12 @@ int finishReads(care_ctx* ctx, hipEvent_t done = nullptr){
     k_hilo<<<gridFor(hiloThreads, 256), dim3(256), 0, st>>>(ctx->enc.as<uint32_t>(), ctx->pitch, ctx->len.as<int>(),
                                                                   num_reads, ctx->W, ctx->hilo.as<uint32_t>(),
                                                                   ctx->rcenc.as<uint32_t>());
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(ctx->lenWeight.ensure(num_reads * 4 + 64));
+    k_len_weight<<<gridFor(num_reads, 256), dim3(256), 0, st>>>(ctx->len.as<int>(),
+                                                                ctx->o.use_quality_scores ? ctx->qual.as<uint8_t>() : nullptr,
+                                                                ctx->qdpitch, ctx->qw.as<float>(), num_reads,
+                                                                ctx->lenWeight.as<uint32_t>());
     HIPCHECK(hipGetLastError());
     if(done) HIPCHECK(hipEventRecord(done, st));
     HIPCHECK(hipStreamSynchronize(st));
