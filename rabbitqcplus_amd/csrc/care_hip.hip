@@ -1601,7 +1601,6 @@ __host__ __device__ inline int tileRowWords(int maxLen){ return (maxLen + 15) >>
 // the slot of qStride(maxLen) bytes holds the whole 16-byte-chunked row).
 __device__ __forceinline__ int rcQualityOffset(const MsaParams& p){ return qStride(p.maxLen) - int(p.qpitch); }
 
-template<int G>
 __device__ __forceinline__ void stageQualities(const MsaParams& p, const MsaTile& t, int tn, int tid, int nthreads);
 
 // Stages candidates [tb, tb+tn) of the working list into the LDS tile: one thread per
@@ -1618,47 +1617,19 @@ __device__ __forceinline__ void stageQualities(const MsaParams& p, const MsaTile
 // vec holds (W even, RW and the enc pitch multiples of 4 words: the enc rows, the
 // reverse-complement rows and the tile slots start on 16-byte boundaries) and the group of
 // four words lies inside the row's RW words.
-// Loads go out in groups (G 16-byte or 4G 4-byte loads) before their stores, so a group
-// costs one memory round trip (G = 1 where the registers of a larger group would spill).
-template<int G>
 __device__ __forceinline__ void stageRow(const uint32_t* __restrict__ src, uint32_t* dst, int len, int RW, bool varLen,
                                          bool vec){
-    if constexpr(G == 1){
-        if(!varLen){
-            for(int k = 0; k < RW; k++) dst[k] = src[k];
-            return;
-        }
-        const int nw = min((len + 15) >> 4, RW);
-        int k = 0;
-        if(vec){
-            for(; k < nw && k + 4 <= RW; k += 4)
-                *reinterpret_cast<uint4*>(dst + k) = *reinterpret_cast<const uint4*>(src + k);
-        }
-        for(; k < nw; k++) dst[k] = src[k];
+    if(!varLen){
+        for(int k = 0; k < RW; k++) dst[k] = src[k];
         return;
     }
-    const int nw = varLen ? min((len + 15) >> 4, RW) : RW;
+    const int nw = min((len + 15) >> 4, RW);
+    int k = 0;
     if(vec){
-        // (RW is a multiple of 4: the 16-byte groups cover the nw words and stay in the row)
-        const uint4* s4 = reinterpret_cast<const uint4*>(src);
-        uint4* d4 = reinterpret_cast<uint4*>(dst);
-        const int nv = (nw + 3) >> 2;
-        for(int g = 0; g < nv; g += G){
-            uint4 r[G];
-            #pragma unroll
-            for(int i = 0; i < G; i++) if(g + i < nv) r[i] = s4[g + i];
-            #pragma unroll
-            for(int i = 0; i < G; i++) if(g + i < nv) d4[g + i] = r[i];
-        }
-        return;
+        for(; k < nw && k + 4 <= RW; k += 4)
+            *reinterpret_cast<uint4*>(dst + k) = *reinterpret_cast<const uint4*>(src + k);
     }
-    for(int g = 0; g < nw; g += 4 * G){
-        uint32_t r[4 * G];
-        #pragma unroll
-        for(int i = 0; i < 4 * G; i++) if(g + i < nw) r[i] = src[g + i];
-        #pragma unroll
-        for(int i = 0; i < 4 * G; i++) if(g + i < nw) dst[g + i] = r[i];
-    }
+    for(; k < nw; k++) dst[k] = src[k];
 }
 
 // Whether 16-byte chunk c of a candidate's quality row holds a byte the MSA reads: a
@@ -1668,7 +1639,6 @@ __device__ __forceinline__ bool qualityChunkUsed(int c, int len, bool rc, int qp
     return rc ? (16 * c + 16 > qpitch - len && 16 * c < qpitch) : 16 * c < len;
 }
 
-template<int G>
 __device__ __forceinline__ void stageTile(const MsaParams& p, const AnchorLists& lst, const MsaTile& t, int beg,
                                           int tb, int tn, int tid, int nthreads){
     const int W = p.W;
@@ -1684,68 +1654,33 @@ __device__ __forceinline__ void stageTile(const MsaParams& p, const AnchorLists&
         // the oriented row (the enc pitch holds at least RW words)
         const uint32_t* src = orient == 1 ? p.enc + p.pitch * id : p.rcenc + uint64_t(id) * uint64_t(2 * W);
         const int RW = tileRowWords(p.maxLen);
-        stageRow<G>(src, t.rows + q * 2 * W, t.len[q], RW, p.varLen != 0, (W & 1) == 0 && (RW & 3) == 0 && (p.pitch & 3) == 0);
+        stageRow(src, t.rows + q * 2 * W, t.len[q], RW, p.varLen != 0, (W & 1) == 0 && (RW & 3) == 0 && (p.pitch & 3) == 0);
     }
     if(!p.useQ) return;
     __syncthreads();
-    stageQualities<G>(p, t, tn, tid, nthreads);
+    stageQualities(p, t, tn, tid, nthreads);
 }
 
 // Quality rows of the tile's tn candidates (ids and orientations already in the tile).
-template<int G>
 __device__ __forceinline__ void stageQualities(const MsaParams& p, const MsaTile& t, int tn, int tid, int nthreads){
     const int qs = qStride(p.maxLen);
     const int nc = qs >> 4;              // chunks per row; device rows are qdpitch >= qs bytes
     // u / nc as a multiply-high: exact for u * nc < 2^32
     const uint64_t magic = ((uint64_t(1) << 32) + uint64_t(nc) - 1) / uint64_t(nc);
-    if constexpr(G == 1){
-        for(int u = tid; u < tn * nc; u += nthreads){
-            const int j = int((uint64_t(u) * magic) >> 32);
-            const int c = u - j * nc;
-            if(p.varLen && !qualityChunkUsed(c, t.len[j], t.orient[j] != 1, int(p.qpitch))) continue;
-            const uint4 v = *reinterpret_cast<const uint4*>(p.qual + p.qdpitch * t.id[j] + 16 * c);
-            uint8_t* dst = t.q + j * qs;
-            if(t.orient[j] == 1){
-                *reinterpret_cast<uint4*>(dst + 16 * c) = v;
-            }else{
-                // byte s of the row goes to qs - 1 - s
-                uint4 r;
-                r.x = __builtin_bswap32(v.w); r.y = __builtin_bswap32(v.z);
-                r.z = __builtin_bswap32(v.y); r.w = __builtin_bswap32(v.x);
-                *reinterpret_cast<uint4*>(dst + qs - 16 * (c + 1)) = r;
-            }
-        }
-        return;
-    }
-    // G chunks per thread in flight before their stores
-    for(int base = tid; base < tn * nc; base += G * nthreads){
-        uint4 v[G];
-        int doff[G];           // byte offset of the chunk's slot in t.q, or -1
-        bool rcv[G];
-        #pragma unroll
-        for(int i = 0; i < G; i++){
-            const int u = base + i * nthreads;
-            doff[i] = -1;
-            rcv[i] = false;
-            v[i] = make_uint4(0u, 0u, 0u, 0u);
-            if(u >= tn * nc) continue;
-            const int j = int((uint64_t(u) * magic) >> 32);
-            const int c = u - j * nc;
-            if(p.varLen && !qualityChunkUsed(c, t.len[j], t.orient[j] != 1, int(p.qpitch))) continue;
-            rcv[i] = t.orient[j] != 1;
-            // a reverse-complement chunk: byte s of the row goes to qs - 1 - s
-            doff[i] = j * qs + (rcv[i] ? qs - 16 * (c + 1) : 16 * c);
-            v[i] = *reinterpret_cast<const uint4*>(p.qual + p.qdpitch * t.id[j] + 16 * c);
-        }
-        #pragma unroll
-        for(int i = 0; i < G; i++){
-            if(doff[i] < 0) continue;
-            uint4 r = v[i];
-            if(rcv[i]){
-                r.x = __builtin_bswap32(v[i].w); r.y = __builtin_bswap32(v[i].z);
-                r.z = __builtin_bswap32(v[i].y); r.w = __builtin_bswap32(v[i].x);
-            }
-            *reinterpret_cast<uint4*>(t.q + doff[i]) = r;
+    for(int u = tid; u < tn * nc; u += nthreads){
+        const int j = int((uint64_t(u) * magic) >> 32);
+        const int c = u - j * nc;
+        if(p.varLen && !qualityChunkUsed(c, t.len[j], t.orient[j] != 1, int(p.qpitch))) continue;
+        const uint4 v = *reinterpret_cast<const uint4*>(p.qual + p.qdpitch * t.id[j] + 16 * c);
+        uint8_t* dst = t.q + j * qs;
+        if(t.orient[j] == 1){
+            *reinterpret_cast<uint4*>(dst + 16 * c) = v;
+        }else{
+            // byte s of the row goes to qs - 1 - s
+            uint4 r;
+            r.x = __builtin_bswap32(v.w); r.y = __builtin_bswap32(v.z);
+            r.z = __builtin_bswap32(v.y); r.w = __builtin_bswap32(v.x);
+            *reinterpret_cast<uint4*>(dst + qs - 16 * (c + 1)) = r;
         }
     }
 }
@@ -1757,52 +1692,74 @@ struct LaneCand {
     float w;
 };
 
-// stageTile for candidates held in lanes: lane tb+q stages candidate tb+q's oriented 2-bit
-// row into slot q, and the quality chunks take their candidate's id and orientation from
-// its lane (ds_bpermute, every lane active), so the row and quality loads are independent.
-// Same rows and qualities as stageTile; the caller reads shift, length and weight from the
-// lanes (the tile's metadata arrays are not written).
-template<int G>
+// Rows of the tile's tn candidates (held in lanes tb..tb+tn-1) in units of T (1, 2 or 4
+// words), spread over the lanes; a row's units past its candidate's length are left out when
+// reads differ in length.
+template<class T>
+__device__ __forceinline__ void stageRowUnits(const MsaParams& p, const MsaTile& t, const LaneCand& c, int tb, int tn, int RW,
+                                              int lane){
+    constexpr int UW = int(sizeof(T) / 4);
+    const int per = RW / UW;
+    const uint64_t magic = ((uint64_t(1) << 32) + uint64_t(per) - 1) / uint64_t(per);     // u / per, exact here
+    const int total = tn * per;
+    constexpr int G = 2;
+    for(int base = 0; base < total; base += G * kWave){
+        T v[G];
+        int at[G];
+        #pragma unroll
+        for(int i = 0; i < G; i++){
+            const int u = base + i * kWave + lane;
+            const int j = min(int((uint64_t(u) * magic) >> 32), tn - 1);
+            const int k = u - j * per;
+            const uint32_t id = uint32_t(__builtin_amdgcn_ds_bpermute(4 * (tb + j), int(c.id)));
+            const int orient = __builtin_amdgcn_ds_bpermute(4 * (tb + j), c.orient);
+            const int len = p.varLen ? __builtin_amdgcn_ds_bpermute(4 * (tb + j), c.len) : RW * 16;
+            const bool ok = u < total && 16 * UW * k < len;
+            at[i] = ok ? j * 2 * p.W + k * UW : -1;
+            const uint32_t* src = orient == 1 ? p.enc + p.pitch * id : p.rcenc + uint64_t(id) * uint64_t(2 * p.W);
+            v[i] = T{};
+            if(ok) v[i] = *reinterpret_cast<const T*>(src + k * UW);
+        }
+        #pragma unroll
+        for(int i = 0; i < G; i++) if(at[i] >= 0) *reinterpret_cast<T*>(t.rows + at[i]) = v[i];
+    }
+}
+
+// Stages candidates tb..tb+tn-1 of a chunk held in lanes: oriented 2-bit rows and quality
+// chunks, all spread over the 64 lanes with their candidate's id, orientation and length taken
+// from its lane (ds_bpermute, every lane active), so that a tile costs one memory round trip
+// for its rows and one for its qualities (G 16-byte loads per lane in flight), where one lane
+// copying a whole row, and reading its list entry per tile, cost four to six. With the grouped
+// slots and the mixed-precision adds of buildMsaWave, k_msa_wave went 10.3 -> 8.6 ms on 1.03M
+// reads of 100..250 bases, 6.5 -> 5.9 ms on 500,000 pairs of 150. The caller reads shift, length and weight from the
+// lanes (the tile's metadata arrays are not written). A reverse-complement candidate reads
+// the pitch-wide quality row reversed (reverseQualitiesOfRCAlignments,
+// include/corrector.hpp:1227-1239): its chunks are byte-reversed in registers and stored
+// mirrored, so that position pos of the reversed row sits at rcQualityOffset + pos.
+template<int G, bool OWNROW>
 __device__ __forceinline__ void stageTileLanes(const MsaParams& p, const MsaTile& t, const LaneCand& c, int tb, int tn,
                                                int lane){
     const int W = p.W;
-    const int q = lane - tb;
-    if(q >= 0 && q < tn){
-        const uint32_t* src = c.orient == 1 ? p.enc + p.pitch * c.id : p.rcenc + uint64_t(c.id) * uint64_t(2 * W);
-        const int RW = tileRowWords(p.maxLen);
-        stageRow<G>(src, t.rows + q * 2 * W, c.len, RW, p.varLen != 0, (W & 1) == 0 && (RW & 3) == 0 && (p.pitch & 3) == 0);
+    const int RW = tileRowWords(p.maxLen);
+    // the enc rows, the reverse-complement rows and the tile slots start on boundaries of the unit
+    const bool vec = (W & 1) == 0 && (RW & 3) == 0 && (p.pitch & 3) == 0;
+    if constexpr(OWNROW){
+        // without qualities a tile is a whole chunk: each lane copies its own candidate's row
+        const int q = lane - tb;
+        if(q >= 0 && q < tn){
+            const uint32_t* src = c.orient == 1 ? p.enc + p.pitch * c.id : p.rcenc + uint64_t(c.id) * uint64_t(2 * W);
+            stageRow(src, t.rows + q * 2 * W, c.len, RW, p.varLen != 0, vec);
+        }
+        return;
     }
+    if(vec) stageRowUnits<uint4>(p, t, c, tb, tn, RW, lane);
+    else if((RW & 1) == 0 && (p.pitch & 1) == 0) stageRowUnits<uint2>(p, t, c, tb, tn, RW, lane);
+    else stageRowUnits<uint32_t>(p, t, c, tb, tn, RW, lane);
     if(!p.useQ) return;
     const int qs = qStride(p.maxLen);
     const int nc = qs >> 4;              // chunks per row; device rows are qdpitch >= qs bytes
     const uint64_t magic = ((uint64_t(1) << 32) + uint64_t(nc) - 1) / uint64_t(nc);   // u / nc, exact here
     const int total = tn * nc;
-    if constexpr(G == 1){
-        for(int base = 0; base < total; base += kWave){
-            const int u = base + lane;
-            const int j = min(int((uint64_t(u) * magic) >> 32), tn - 1);
-            const uint32_t id = uint32_t(__builtin_amdgcn_ds_bpermute(4 * (tb + j), int(c.id)));
-            const int orient = __builtin_amdgcn_ds_bpermute(4 * (tb + j), c.orient);
-            // reads of one length use every chunk (fixed length: no test, no third permute)
-            const int len = p.varLen ? __builtin_amdgcn_ds_bpermute(4 * (tb + j), c.len) : int(p.qpitch);
-            if(u < total && (!p.varLen || qualityChunkUsed(u - j * nc, len, orient != 1, int(p.qpitch)))){
-                const int ch = u - j * nc;
-                const uint4 v = *reinterpret_cast<const uint4*>(p.qual + p.qdpitch * id + 16 * ch);
-                uint8_t* dst = t.q + j * qs;
-                if(orient == 1){
-                    *reinterpret_cast<uint4*>(dst + 16 * ch) = v;
-                }else{
-                    // byte s of the row goes to qs - 1 - s
-                    uint4 r;
-                    r.x = __builtin_bswap32(v.w); r.y = __builtin_bswap32(v.z);
-                    r.z = __builtin_bswap32(v.y); r.w = __builtin_bswap32(v.x);
-                    *reinterpret_cast<uint4*>(dst + qs - 16 * (ch + 1)) = r;
-                }
-            }
-        }
-        return;
-    }
-    // G chunks per lane in flight before their stores (one memory round trip per group)
     for(int base = 0; base < total; base += G * kWave){
         uint4 v[G];
         int doff[G];           // byte offset of the chunk's slot in t.q, or -1
@@ -1820,7 +1777,8 @@ __device__ __forceinline__ void stageTileLanes(const MsaParams& p, const MsaTile
             rcv[i] = orient != 1;
             // a reverse-complement chunk: byte s of the row goes to qs - 1 - s
             doff[i] = ok ? j * qs + (rcv[i] ? qs - 16 * (ch + 1) : 16 * ch) : -1;
-            v[i] = ok ? *reinterpret_cast<const uint4*>(p.qual + p.qdpitch * id + 16 * ch) : make_uint4(0u, 0u, 0u, 0u);
+            v[i] = make_uint4(0u, 0u, 0u, 0u);
+            if(ok) v[i] = *reinterpret_cast<const uint4*>(p.qual + p.qdpitch * id + 16 * ch);
         }
         #pragma unroll
         for(int i = 0; i < G; i++){
@@ -1877,7 +1835,7 @@ __device__ bool buildMsa(const MsaParams& p, MsaShared& sh, uint64_t a, int La, 
     for(int tb = 0; tb < nk; tb += T){
         const int tn = min(T, nk - tb);
         __syncthreads();   // previous tile fully consumed
-        stageTile<1>(p, listsOf(p), t, beg, tb, tn, threadIdx.x, kBlock);
+        stageTile(p, listsOf(p), t, beg, tb, tn, threadIdx.x, kBlock);
         __syncthreads();
         for(int c = threadIdx.x; c < ncol; c += kBlock){
             int n0 = cnt[4 * c + 0], n1 = cnt[4 * c + 1], n2 = cnt[4 * c + 2], n3 = cnt[4 * c + 3];
@@ -2238,6 +2196,8 @@ __device__ __forceinline__ int waveReduce(int v, Op op, int identity){
     return __builtin_amdgcn_readlane(v, 63);
 }
 
+typedef _Float16 Half4 __attribute__((ext_vector_type(4)));
+
 // pointers into LDS (address space 3, 32-bit)
 typedef const __attribute__((address_space(3))) uint32_t* LdsU32;
 typedef const __attribute__((address_space(3))) uint8_t* LdsU8;
@@ -2322,30 +2282,30 @@ __device__ __forceinline__ bool buildMsaWave(const MsaParams& p, const AnchorLis
     const int T = p.tile;
     const int qs = qStride(p.maxLen);
     const int qrc = rcQualityOffset(p);
-    for(int tb = 0; tb < nk; tb += T){
-        const int tn = min(T, nk - tb);
-        __syncthreads();
-        // two loads in flight per lane from 3 column slots on (at 2 slots the 8-wave budget
-        // leaves no room)
-        constexpr int G = KC >= 3 ? 2 : 1;
-        if(inLanes) stageTileLanes<G>(p, t, lc, tb, tn, lane);
-        else stageTile<G>(p, lst, t, beg, tb, tn, lane, kWave);
-        __syncthreads();
-        // lane src+q holds candidate tb+q's shift, length, weight and orientation; the loop
-        // below reads them with readlane (no LDS round trip per candidate)
-        int mShift = 0, mLen = 0, mRc = 0, src = tb;
-        float mW = 0.0f;
-        if(inLanes){
-            mShift = lc.shift; mLen = lc.len; mW = lc.w; mRc = lc.orient != 1;
-        }else{
-            src = 0;
-            if(lane < tn){ mShift = t.shift[lane]; mLen = t.len[lane]; mW = t.w[lane]; mRc = t.orient[lane] != 1; }
+    // chunks of 64 candidates: lane i holds candidate i of the chunk
+    for(int cb = 0; cb < nk; cb += kWave){
+    LaneCand c = lc;
+    if(!inLanes){
+        c = LaneCand{};
+        const int d = beg + cb + lane;
+        if(cb + lane < nk){
+            c.id = lst.kId[d]; c.shift = lst.kShift[d]; c.len = lst.kLen[d]; c.orient = lst.kOrient[d]; c.w = lst.kW[d];
         }
+    }
+    const int cn = min(kWave, nk - cb);
+    for(int tb = 0; tb < cn; tb += T){
+        const int tn = min(T, cn - tb);
+        __syncthreads();
+        stageTileLanes<(KC <= 4 ? 4 : 2), QM == 0>(p, t, c, tb, tn, lane);
+        __syncthreads();
+        // lane tb+j holds candidate j's shift, length, weight and orientation; the loop below
+        // reads them with readlane (no LDS round trip per candidate)
+        const int mRc = c.orient != 1;
         for(int j = 0; j < tn; j++){
-            const int cs = off + __builtin_amdgcn_readlane(mShift, src + j);   // slot column of its first base
-            const int ln = __builtin_amdgcn_readlane(mLen, src + j);
-            const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mW), src + j));
-            const bool rc = __builtin_amdgcn_readlane(mRc, src + j) != 0;
+            const int cs = off + __builtin_amdgcn_readlane(c.shift, tb + j);   // slot column of its first base
+            const int ln = __builtin_amdgcn_readlane(c.len, tb + j);
+            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.w * 0x1p24f), tb + j));
+            const bool rc = __builtin_amdgcn_readlane(mRc, tb + j) != 0;
             // slots holding its columns (AO: those under the anchor; lanes past the anchor
             // end add to columns that are never read)
             const int k0 = (AO ? max(cs, 0) : cs) >> 6;
@@ -2355,34 +2315,55 @@ __device__ __forceinline__ bool buildMsaWave(const MsaParams& p, const AnchorLis
             const int pos0 = lane - cs;
             const int sA = 30 - 2 * (pos0 & 15);
             // LDS addresses of slot 0's base word and quality byte, kept in registers (the
-            // compiler would otherwise rebuild them inside every slot's branch; the empty asm
-            // statement emits no instruction). Slot k reads rowp[4k] and qp[64k], which lie
-            // in candidate j's row whenever the slot's position is inside the candidate.
+            // compiler would otherwise rebuild them for every slot; the empty asm statement
+            // emits no instruction). Slot k reads rowp[4k] and qp[64k].
             LdsU32 rowp = (LdsU32)(t.rows) + (j * RS + (pos0 >> 4));
             LdsU8 qp = (LdsU8)(t.q) + (j * qs + (rc ? qrc : 0) + pos0);
             asm volatile("" : "+v"(rowp), "+v"(qp));
+            // Slots go in groups without a branch per slot: the base word, the quality byte and
+            // the weight lookup of a group's slots are in flight together (two LDS round trips
+            // per group; one slot at a time they cost two each, and the kernel waited for
+            // them). A lane outside the candidate reads whatever lies there (its addresses
+            // stay inside the workgroup's LDS, see waveMsaLdsBytes) and adds nothing: its
+            // one-hot factors and its count are 0.
+            constexpr int GS = KC <= 3 ? KC : 2;
             #pragma unroll
-            for(int k = 0; k < KC; k++){
-                if(k < k0 || k > k1) continue;        // wave-uniform
-                const int pos = pos0 + kWave * k;
-                if(unsigned(pos) < unsigned(ln)){
-                    const int b = int((rowp[4 * k] >> sA) & 3u);
-                    const float x = wj * (useQ ? t.qw[qp[kWave * k]] : 1.0f);
-                    // inc holds 1 in the 16-bit field of base b, so bytes 0 and 2 of its
-                    // halves are the one-hot factors of A, C (low half) and G, T (high half).
-                    // fma(x, 1, w) rounds w + x exactly like the add and fma(x, 0, w) = w (no
-                    // weight is ever -0.0: weights start at +0.0f and add finite products),
-                    // so each weight is the sum of its base's x in list order, branch-free.
-                    const uint64_t inc = uint64_t(1) << (16 * b);
-                    const uint32_t incLo = uint32_t(inc), incHi = uint32_t(inc >> 32);
-                    m.w[k][0] = __builtin_fmaf(x, float(incLo & 0xFFu), m.w[k][0]);
-                    m.w[k][1] = __builtin_fmaf(x, float((incLo >> 16) & 0xFFu), m.w[k][1]);
-                    m.w[k][2] = __builtin_fmaf(x, float(incHi & 0xFFu), m.w[k][2]);
-                    m.w[k][3] = __builtin_fmaf(x, float((incHi >> 16) & 0xFFu), m.w[k][3]);
+            for(int kg = 0; kg < KC; kg += GS){
+                if(kg > k1 || kg + GS <= k0) continue;        // wave-uniform
+                uint32_t word[GS];
+                float x[GS];
+                #pragma unroll
+                for(int g = 0; g < GS; g++) word[g] = rowp[4 * (kg + g)];
+                if(useQ){
+                    uint32_t qv[GS];
+                    #pragma unroll
+                    for(int g = 0; g < GS; g++) qv[g] = qp[kWave * (kg + g)];
+                    #pragma unroll
+                    for(int g = 0; g < GS; g++) x[g] = ws * t.qw[qv[g]];
+                }else{
+                    #pragma unroll
+                    for(int g = 0; g < GS; g++) x[g] = ws;
+                }
+                #pragma unroll
+                for(int g = 0; g < GS; g++){
+                    const int k = kg + g;
+                    const uint32_t one = unsigned(pos0 + kWave * k) < unsigned(ln) ? 1u : 0u;
+                    const int b = int((word[g] >> sA) & 3u);
+                    // inc holds 1 in the 16-bit field of base b: read as half floats its four
+                    // fields are 2^-24 for b and 0 for the others, so one mixed-precision fma
+                    // per base adds the base's weight: x carries a factor of 2^24 (exact), and
+                    // fma(x, 2^-24, w) rounds w + x exactly like the add and fma(x, 0, w) = w
+                    // (no weight is ever -0.0: weights start at +0.0f and add finite
+                    // products). Each weight is the sum of its base's x in list order.
+                    const uint64_t inc = uint64_t(one) << (16 * b);
+                    const Half4 hot = __builtin_bit_cast(Half4, inc);
+                    #pragma unroll
+                    for(int q = 0; q < 4; q++) m.w[k][q] = __builtin_fmaf(x[g], float(hot[q]), m.w[k][q]);
                     m.cnt[k] += inc;
                 }
             }
         }
+    }
     }
     // consensus and support (src/msa.cpp:135-157)
     m.cons = 0;
@@ -3164,7 +3145,7 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
 
 template<int KC, bool AO, int QM>
 __global__ void __launch_bounds__(kWave)
-__attribute__((amdgpu_waves_per_eu(AO && KC <= 3 ? 7 : (KC <= 8 ? 4 : 2))))
+__attribute__((amdgpu_waves_per_eu(AO && KC <= 3 ? 6 : (AO && KC <= 4 ? 5 : (KC <= 8 ? 4 : 2)))))
 k_msa_wave(MsaParams p){
     extern __shared__ uint8_t smem[];
     __shared__ float sQw[256];
@@ -3829,15 +3810,18 @@ int waveMsaAnchorSlots(int maxLen){
     return 0;
 }
 
-// Candidates per LDS tile of the one-wavefront MSA. With qualities (220 bytes per
-// candidate at 150 bp) 20 keeps the workgroup near 6 KB, so about 26 one-wavefront
-// workgroups fit a compute unit's LDS (the anchor-column kernels with at most 3 register
-// columns per lane are built for 7 waves per SIMD); without qualities 64 fit in less.
-int defaultWaveMsaTile(bool useQ){ return useQ ? 20 : 64; }
+// Candidates per LDS tile of the one-wavefront MSA. With qualities 16: 220 bytes per
+// candidate at 150 bases, 340 at 250, where the workgroup's LDS then lets 5 waves per SIMD
+// reside (k_msa_wave at 12/16/20/24 candidates: 9.4/8.7/10.4/10.9 ms on 1.03M reads of
+// 100..250 bases, 6.3/5.9/6.0/6.2 ms on 500,000 pairs of 150); without qualities a whole
+// chunk of 64 fits in less (16/32/64: 1.68/1.62/1.58 ms on 594,000 reads of 101 bases).
+int defaultWaveMsaTile(bool useQ){ return useQ ? 16 : 64; }
 
-// dynamic LDS of k_msa_wave: tile region + anchor-column supports
+// dynamic LDS of k_msa_wave: tile region + anchor-column supports + 192 bytes: lanes outside
+// a candidate read up to 191 positions past its row (a group of 3 slots), from the last row
+// of a tile without supports behind it up to here; before the first row lies the weight table
 size_t waveMsaLdsBytes(int tile, int W, int maxLen, bool useQ, bool seam, int maxCols){
-    return waveTileRegion(tile, W, maxLen, useQ, seam, maxCols) + size_t(maxLen) * 4 + 16;
+    return waveTileRegion(tile, W, maxLen, useQ, seam, maxCols) + size_t(maxLen) * 4 + 16 + 192;
 }
 
 // Candidates per LDS tile: as many as fit next to the column arrays in ~40 KB, 16..64.
