@@ -326,29 +326,61 @@ __global__ void k_iota(uint32_t* v, uint64_t n){
 }
 
 // Buckets that survive the 2..threshold rule (include/groupbykey.hpp:176-215).
-__global__ void k_count_kept(const uint32_t* counts, const int* numRuns, int thr, uint32_t* kept){
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= *numRuns) return;
-    const uint32_t c = counts[i];
-    if(c >= 2 && c <= uint32_t(thr)) atomicAdd(kept, 1u);
+// Table build over a group of maps at once: items are (map, read), a key is the signature with
+// the map's number within the group above its `shift` bits (groups of one map: the signature),
+// so one stable sort, one run-length encode and one scan serve every map of the group.
+__global__ void k_tag_keys(const uint64_t* __restrict__ sig, uint64_t n, uint64_t items, int shift, uint64_t* __restrict__ keys,
+                           uint32_t* __restrict__ ids){
+    FOR_GRID(i, items){
+        const uint64_t m = i / n;
+        keys[i] = sig[i] | (m << shift);
+        ids[i] = uint32_t(i - m * n);
+    }
 }
 
-__global__ void k_insert(const uint64_t* keys, const uint32_t* counts, const uint32_t* offsets, const int* numRuns,
-                         int thr, Slot* slots, uint32_t capMask){
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= *numRuns) return;
-    const uint32_t c = counts[i];
-    if(c < 2 || c > uint32_t(thr)) return;
-    const uint64_t key = keys[i];
-    uint32_t h = uint32_t(fmix64(key)) & capMask;
-    // keys are unique, so claiming an empty slot (count 0 -> c) is the only race
-    for(;;){
-        if(atomicCAS(&slots[h].count, 0u, c) == 0u){
-            slots[h].key = key;
-            slots[h].offset = offsets[i];
-            return;
-        }
-        h = (h + 1) & capMask;
+constexpr int kGroupMaps = 64;      // maps per group at most
+__device__ __forceinline__ int mapOfKey(uint64_t key, int shift){ return shift < 64 ? int(key >> shift) : 0; }
+
+// Kept buckets (2..thr values) per map of the group.
+__global__ void __launch_bounds__(256) k_count_kept(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ counts,
+                                                    const int* __restrict__ numRuns, int thr, int shift,
+                                                    uint32_t* __restrict__ kept){
+    __shared__ uint32_t sum[kGroupMaps];
+    if(threadIdx.x < kGroupMaps) sum[threadIdx.x] = 0;
+    __syncthreads();
+    const int runs = *numRuns;
+    FOR_GRID(i, runs){
+        const uint32_t c = counts[i];
+        if(c >= 2 && c <= uint32_t(thr)) atomicAdd(&sum[mapOfKey(keys[i], shift)], 1u);
+    }
+    __syncthreads();
+    if(threadIdx.x < kGroupMaps && sum[threadIdx.x]) atomicAdd(&kept[threadIdx.x], sum[threadIdx.x]);
+}
+
+// Empties the tables of maps [m0, m0 + gridDim.y).
+__global__ void k_clear_slots(Slot* const* slots, const uint32_t* caps, int m0){
+    const int m = m0 + int(blockIdx.y);
+    uint4* s = reinterpret_cast<uint4*>(slots[m]);
+    for(uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < caps[m]; i += gridDim.x * blockDim.x)
+        s[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+__global__ void k_insert(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ counts,
+                         const uint32_t* __restrict__ offsets, const int* __restrict__ numRuns, int thr, int shift, uint64_t n,
+                         Slot* const* slots, const uint32_t* caps, int m0){
+    FOR_GRID(i, *numRuns){
+        const uint32_t c = counts[i];
+        if(c < 2 || c > uint32_t(thr)) continue;
+        const int m = mapOfKey(keys[i], shift);
+        const uint64_t key = shift < 64 ? keys[i] & ((uint64_t(1) << shift) - 1) : keys[i];
+        const uint32_t offset = uint32_t(uint64_t(offsets[i]) - uint64_t(m) * n);     // every map has n items
+        Slot* table = slots[m0 + m];
+        const uint32_t capMask = caps[m0 + m] - 1;
+        uint32_t h = uint32_t(fmix64(key)) & capMask;
+        // keys are unique, so claiming an empty slot (count 0 -> c) is the only race
+        while(atomicCAS(&table[h].count, 0u, c) != 0u) h = (h + 1) & capMask;
+        table[h].key = key;
+        table[h].offset = offset;
     }
 }
 
@@ -3621,7 +3653,7 @@ struct care_ctx {
     // batch working memory
     DBuf raw, uniq, offsets, ids, anchorOf, best, dbg, paired;
     DBuf kId, kShift, kLen, kNops, kOvl, kW, kOrient, kPaired;
-    DBuf slots, recBytes, recOff, recOff64, outBuf, info, msaDbg, counters, scanTmp, scratch, candOver, alignOver, lenWeight;
+    DBuf slots, recBytes, recOff, recOff64, outBuf, info, msaDbg, counters, scanTmp, scratch, candOver, alignOver, lenWeight, tableTmp;
     // learned seam: classifier (bfloat16 weights then float biases) and feature output
     DBuf seam, featBuf, metaBuf;
     // pinned host words: record bytes (u64) and the error flag (i32) of the last pass
@@ -3701,79 +3733,103 @@ int resultsPerMapThreshold(float coverage){
     return std::max(10, result);
 }
 
+// Items (map, read) that one group of the table build sorts together, unless one map has more.
+// Small read sets are bound by launches and by the host's wait for the kept counts: a table
+// build (k = 20) at 6,000 / 400,000 / 1.0M / 4.0M reads of 150 bases took 4.5 / 12.0 / 18.2 /
+// 40.1 ms map by map with buffers of its own, 0.34 / 3.5 / 8.2 / 33.0 ms in groups. 2^24 items
+// keep the sort's passes at the card's bandwidth and the workspace below 1 GB.
+constexpr uint64_t kGroupItems = uint64_t(1) << 24;
+
 int buildTables(care_ctx* ctx){
     const uint64_t n = ctx->n;
     const int M = ctx->M;
     hipStream_t st = ctx->stream;
-    DBuf iota, keysOut, uniqKeys, runCounts, runOffsets, numRuns, kept, temp;
-    auto cleanup = [&](){ iota.release(); keysOut.release(); uniqKeys.release(); runCounts.release();
-                          runOffsets.release(); numRuns.release(); kept.release(); temp.release(); };
-    struct Guard { decltype(cleanup)& f; ~Guard(){ f(); } } guard{cleanup};
-
-    HIPCHECK(ctx->values.ensure(std::max<uint64_t>(1, n) * M * sizeof(uint32_t)));
-    HIPCHECK(iota.ensure(std::max<uint64_t>(1, n) * sizeof(uint32_t)));
-    HIPCHECK(keysOut.ensure(std::max<uint64_t>(1, n) * sizeof(uint64_t)));
-    HIPCHECK(uniqKeys.ensure(std::max<uint64_t>(1, n) * sizeof(uint64_t)));
-    HIPCHECK(runCounts.ensure(std::max<uint64_t>(1, n) * sizeof(uint32_t)));
-    HIPCHECK(runOffsets.ensure(std::max<uint64_t>(1, n) * sizeof(uint32_t)));
-    HIPCHECK(numRuns.ensure(sizeof(int)));
-    HIPCHECK(kept.ensure(sizeof(uint32_t)));
-    if(n) k_iota<<<gridFor(n, 256), dim3(256), 0, st>>>(iota.as<uint32_t>(), n);
-    HIPCHECK(hipGetLastError());
+    const int sigBits = 2 * ctx->k;
+    // maps per group: their number must fit above the signature's bits
+    int group = int(std::min<uint64_t>({uint64_t(M), uint64_t(kGroupMaps), std::max<uint64_t>(1, kGroupItems / std::max<uint64_t>(1, n))}));
+    if(sigBits > 58) group = 1;
+    const int shift = group > 1 ? sigBits : 64;
+    int endBit = sigBits;
+    while(group > 1 && (1 << (endBit - sigBits)) < group) endBit++;
+    const uint64_t items = std::max<uint64_t>(1, uint64_t(group) * n);
 
     size_t tb1 = 0, tb2 = 0, tb3 = 0;
-    const int endBit = 2 * ctx->k;
     HIPCHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb1, (const uint64_t*)nullptr, (uint64_t*)nullptr,
-                                                (const uint32_t*)nullptr, (uint32_t*)nullptr, int(n), 0, endBit, st));
+                                                (const uint32_t*)nullptr, (uint32_t*)nullptr, int(items), 0, endBit, st));
     HIPCHECK(hipcub::DeviceRunLengthEncode::Encode(nullptr, tb2, (const uint64_t*)nullptr, (uint64_t*)nullptr,
-                                                   (uint32_t*)nullptr, (int*)nullptr, int(n), st));
-    HIPCHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb3, (const uint32_t*)nullptr, (uint32_t*)nullptr, int(n), st));
-    HIPCHECK(temp.ensure(std::max({tb1, tb2, tb3, size_t(256)})));
+                                                   (uint32_t*)nullptr, (int*)nullptr, int(items), st));
+    HIPCHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb3, (const uint32_t*)nullptr, (uint32_t*)nullptr, int(items), st));
+    const size_t tempBytes = std::max({tb1, tb2, tb3, size_t(256)});
+    // one workspace, kept by the context for the next reads (its size is bounded by
+    // kGroupItems or one map, about 50 bytes per item)
+    auto up = [](size_t b){ return (b + 255) & ~size_t(255); };
+    const size_t b8 = up(items * 8), b4 = up(items * 4);
+    HIPCHECK(ctx->tableTmp.ensure((group > 1 ? 3 : 2) * b8 + 3 * b4 + 512 + up(tempBytes)));
+    uint8_t* w = ctx->tableTmp.as<uint8_t>();
+    auto take = [&](size_t b){ uint8_t* q = w; w += b; return q; };
+    uint64_t* keysOut = reinterpret_cast<uint64_t*>(take(b8));
+    uint64_t* uniqKeys = reinterpret_cast<uint64_t*>(take(b8));
+    uint64_t* keysIn = group > 1 ? reinterpret_cast<uint64_t*>(take(b8)) : nullptr;
+    uint32_t* idsIn = reinterpret_cast<uint32_t*>(take(b4));
+    uint32_t* runCounts = reinterpret_cast<uint32_t*>(take(b4));
+    uint32_t* runOffsets = reinterpret_cast<uint32_t*>(take(b4));
+    uint32_t* kept = reinterpret_cast<uint32_t*>(take(512));           // kGroupMaps counters, then the run count
+    int* numRuns = reinterpret_cast<int*>(kept + kGroupMaps);
+    void* temp = take(up(tempBytes));
 
-    ctx->slotBufs.resize(M);
-    ctx->caps.assign(M, 0);
-    std::vector<Slot*> ptrs(M, nullptr);
-    for(int m = 0; m < M; m++){
-        const uint64_t* keysIn = ctx->sig.as<uint64_t>() + uint64_t(m) * n;
-        uint32_t* vals = ctx->values.as<uint32_t>() + uint64_t(m) * n;
-        size_t b = temp.bytes;
-        // stable LSD radix sort: equal keys keep ascending read ids
-        HIPCHECK(hipcub::DeviceRadixSort::SortPairs(temp.p, b, keysIn, keysOut.as<uint64_t>(), iota.as<uint32_t>(),
-                                                    vals, int(n), 0, endBit, st));
-        b = temp.bytes;
-        HIPCHECK(hipcub::DeviceRunLengthEncode::Encode(temp.p, b, keysOut.as<uint64_t>(), uniqKeys.as<uint64_t>(),
-                                                       runCounts.as<uint32_t>(), numRuns.as<int>(), int(n), st));
-        b = temp.bytes;
-        HIPCHECK(hipcub::DeviceScan::ExclusiveSum(temp.p, b, runCounts.as<uint32_t>(), runOffsets.as<uint32_t>(),
-                                                  int(n), st));
-        HIPCHECK(hipMemsetAsync(kept.p, 0, sizeof(uint32_t), st));
-        const int grid = int((n + 255) / 256);
-        if(grid){
-            k_count_kept<<<grid, 256, 0, st>>>(runCounts.as<uint32_t>(), numRuns.as<int>(), ctx->thr, kept.as<uint32_t>());
-            HIPCHECK(hipGetLastError());
-        }
-        uint32_t keptHost = 0;
-        HIPCHECK(hipMemcpyAsync(&keptHost, kept.p, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        HIPCHECK(hipStreamSynchronize(st));
-        uint32_t cap = 64;
-        while(cap < 2u * keptHost) cap <<= 1;
-        ctx->caps[m] = cap;
-        HIPCHECK(ctx->slotBufs[m].ensure(size_t(cap) * sizeof(Slot)));
-        HIPCHECK(hipMemsetAsync(ctx->slotBufs[m].p, 0, size_t(cap) * sizeof(Slot), st));
-        if(grid){
-            k_insert<<<grid, 256, 0, st>>>(uniqKeys.as<uint64_t>(), runCounts.as<uint32_t>(), runOffsets.as<uint32_t>(),
-                                           numRuns.as<int>(), ctx->thr, ctx->slotBufs[m].as<Slot>(), cap - 1);
-            HIPCHECK(hipGetLastError());
-        }
-        ptrs[m] = ctx->slotBufs[m].as<Slot>();
-    }
+    HIPCHECK(ctx->values.ensure(std::max<uint64_t>(1, n) * M * sizeof(uint32_t)));
     HIPCHECK(ctx->slotPtrs.ensure(sizeof(Slot*) * kMaxMaps));
     HIPCHECK(ctx->capsDev.ensure(sizeof(uint32_t) * kMaxMaps));
-    std::vector<Slot*> ptrs48(kMaxMaps, nullptr);
-    std::vector<uint32_t> caps48(kMaxMaps, 1);
-    for(int m = 0; m < M; m++){ ptrs48[m] = ptrs[m]; caps48[m] = ctx->caps[m]; }
-    HIPCHECK(hipMemcpyAsync(ctx->slotPtrs.p, ptrs48.data(), sizeof(Slot*) * kMaxMaps, hipMemcpyHostToDevice, st));
-    HIPCHECK(hipMemcpyAsync(ctx->capsDev.p, caps48.data(), sizeof(uint32_t) * kMaxMaps, hipMemcpyHostToDevice, st));
+    ctx->slotBufs.resize(M);
+    ctx->caps.assign(M, 0);
+    std::vector<Slot*> ptrs(kMaxMaps, nullptr);
+    std::vector<uint32_t> caps(kMaxMaps, 1);
+    if(group == 1 && n) k_iota<<<gridFor(n, 256), dim3(256), 0, st>>>(idsIn, n);
+    HIPCHECK(hipGetLastError());
+    for(int m0 = 0; m0 < M; m0 += group){
+        const int g = std::min(group, M - m0);
+        const uint64_t count = uint64_t(g) * n;
+        const uint64_t* sig = ctx->sig.as<uint64_t>() + uint64_t(m0) * n;
+        uint32_t* vals = ctx->values.as<uint32_t>() + uint64_t(m0) * n;
+        if(group > 1 && count){
+            k_tag_keys<<<gridFor(count, 256), dim3(256), 0, st>>>(sig, n, count, shift, keysIn, idsIn);
+            HIPCHECK(hipGetLastError());
+        }
+        // stable LSD radix sort: equal keys keep ascending read ids
+        size_t b = tempBytes;
+        HIPCHECK(hipcub::DeviceRadixSort::SortPairs(temp, b, group > 1 ? keysIn : sig, keysOut, idsIn, vals, int(count), 0, endBit, st));
+        b = tempBytes;
+        HIPCHECK(hipcub::DeviceRunLengthEncode::Encode(temp, b, keysOut, uniqKeys, runCounts, numRuns, int(count), st));
+        b = tempBytes;
+        HIPCHECK(hipcub::DeviceScan::ExclusiveSum(temp, b, runCounts, runOffsets, int(count), st));
+        k_zero_u32<<<1, 64, 0, st>>>(kept, kGroupMaps);
+        HIPCHECK(hipGetLastError());
+        const dim3 grid(uint32_t(std::min<uint64_t>((count + 255) / 256, 8192)));
+        if(count){
+            k_count_kept<<<grid, 256, 0, st>>>(uniqKeys, runCounts, numRuns, ctx->thr, shift, kept);
+            HIPCHECK(hipGetLastError());
+        }
+        uint32_t keptHost[kGroupMaps] = {};
+        HIPCHECK(hipMemcpyAsync(keptHost, kept, size_t(g) * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        HIPCHECK(hipStreamSynchronize(st));
+        for(int m = m0; m < m0 + g; m++){
+            uint32_t cap = 64;
+            while(cap < 2u * keptHost[m - m0]) cap <<= 1;
+            ctx->caps[m] = cap;
+            HIPCHECK(ctx->slotBufs[m].ensure(size_t(cap) * sizeof(Slot)));
+            ptrs[m] = ctx->slotBufs[m].as<Slot>();
+            caps[m] = cap;
+        }
+        HIPCHECK(hipMemcpyAsync(ctx->slotPtrs.p, ptrs.data(), sizeof(Slot*) * kMaxMaps, hipMemcpyHostToDevice, st));
+        HIPCHECK(hipMemcpyAsync(ctx->capsDev.p, caps.data(), sizeof(uint32_t) * kMaxMaps, hipMemcpyHostToDevice, st));
+        k_clear_slots<<<dim3(128, uint32_t(g)), dim3(256), 0, st>>>(ctx->slotPtrs.as<Slot*>(), ctx->capsDev.as<uint32_t>(), m0);
+        HIPCHECK(hipGetLastError());
+        if(count){
+            k_insert<<<grid, 256, 0, st>>>(uniqKeys, runCounts, runOffsets, numRuns, ctx->thr, shift, n,
+                                           ctx->slotPtrs.as<Slot*>(), ctx->capsDev.as<uint32_t>(), m0);
+            HIPCHECK(hipGetLastError());
+        }
+    }
     HIPCHECK(hipStreamSynchronize(st));
     return CARE_OK;
 }
@@ -4968,7 +5024,7 @@ void care_hip_destroy(care_ctx* ctx){
                    &ctx->fqHdrLen, &ctx->fqSeq, &ctx->fqQual, &ctx->mRec, &ctx->mOff, &ctx->mKeyIn, &ctx->mKeyOut,
                    &ctx->mIdxIn, &ctx->mIdxOut, &ctx->mRunBeg, &ctx->mRunEnd, &ctx->mPlan, &ctx->mSize, &ctx->mOutOff,
                    &ctx->mText, &ctx->mErr, &ctx->candSlots, &ctx->candBytes, &ctx->insSize, &ctx->insOff,
-                   &ctx->insSrc, &ctx->hqAnchor, &ctx->seeds, &ctx->alignOver, &ctx->lenWeight, &ctx->pipeOut[0], &ctx->pipeOut[1]}){
+                   &ctx->insSrc, &ctx->hqAnchor, &ctx->seeds, &ctx->alignOver, &ctx->lenWeight, &ctx->tableTmp, &ctx->pipeOut[0], &ctx->pipeOut[1]}){
         b->release();
     }
     if(ctx->fusedExec) (void)hipGraphExecDestroy(ctx->fusedExec);
@@ -6330,7 +6386,9 @@ static int care_hip_inspect_reads_body(care_ctx* ctx, uint64_t first, uint64_t n
 }
 
 // Resolves every read's bucket per map (after the tables are built or loaded).
-static int resolveBuckets(care_ctx* ctx){
+// built: the tables were built here, so the values of map 0 are all reads in the order of their
+// map-0 signatures (a loaded file holds the kept buckets' values only).
+static int resolveBuckets(care_ctx* ctx, bool built){
     hipStream_t st = ctx->stream;
     const uint64_t total = ctx->n * uint64_t(ctx->M);
     HIPCHECK(ctx->bucketOf.ensure(total * sizeof(uint2)));
@@ -6339,7 +6397,11 @@ static int resolveBuckets(care_ctx* ctx){
                                                                     ctx->capsDev.as<uint32_t>(), ctx->bucketOf.as<uint2>());
     HIPCHECK(hipGetLastError());
     // processing order: reads sorted by their map-0 signature (reads that share it overlap)
-    {
+    if(built){
+        HIPCHECK(ctx->order.ensure(ctx->n * 4));
+        if(ctx->n) HIPCHECK(hipMemcpyAsync(ctx->order.p, ctx->values.p, ctx->n * 4, hipMemcpyDeviceToDevice, st));
+        HIPCHECK(hipStreamSynchronize(st));
+    }else{
         struct Tmp { DBuf keys, ids; ~Tmp(){ keys.release(); ids.release(); } } tmp;
         const uint64_t n = ctx->n;
         HIPCHECK(ctx->order.ensure(n * 4));
@@ -6372,7 +6434,7 @@ static int care_hip_build_tables_body(care_ctx* ctx, int* maps_built){
     HIPCHECK(hipGetLastError());
     int rc = buildTables(ctx);
     if(rc != CARE_OK) return rc;
-    rc = resolveBuckets(ctx);
+    rc = resolveBuckets(ctx, true);
     if(rc != CARE_OK) return rc;
     ctx->hasTables = true;
     if(maps_built) *maps_built = ctx->M;
@@ -6527,7 +6589,7 @@ static int care_hip_load_tables_body(care_ctx* ctx, const char* path, int* maps_
     HIPCHECK(hipMemcpy(ctx->slotPtrs.p, ptrs48.data(), sizeof(Slot*) * kMaxMaps, hipMemcpyHostToDevice));
     HIPCHECK(hipMemcpy(ctx->capsDev.p, caps48.data(), sizeof(uint32_t) * kMaxMaps, hipMemcpyHostToDevice));
     HIPCHECK(hipStreamSynchronize(st));
-    const int rc = resolveBuckets(ctx);
+    const int rc = resolveBuckets(ctx, false);
     if(rc != CARE_OK) return rc;
     ctx->hasTables = true;
     if(maps_loaded) *maps_loaded = M;
