@@ -712,8 +712,13 @@ k_candidates_over(CandParams p, const uint32_t* __restrict__ over, const uint32_
 // Sum of the per-anchor gathered-value counts of a batch into the pass counter: each
 // block sums kAddPerBlock counts and adds them with one atomic.
 constexpr int kAddPerBlock = 16 * kBlock;
+constexpr int kStatusWords = 12;     // of a pipelined batch (slotStatus)
 
-__global__ void k_add_gathered(const uint32_t* __restrict__ gath, int B, unsigned long long* __restrict__ total){
+__global__ void k_add_gathered(const uint32_t* __restrict__ first, int B, unsigned long long* __restrict__ firstTotal,
+                               const uint32_t* __restrict__ second, unsigned long long* __restrict__ secondTotal){
+    // blockIdx.y: which of the two sums (grids of one row: the first)
+    const uint32_t* __restrict__ gath = blockIdx.y ? second : first;
+    unsigned long long* __restrict__ total = blockIdx.y ? secondTotal : firstTotal;
     __shared__ unsigned long long part[kBlock / kWave];
     unsigned long long s = 0;
     const int lo = blockIdx.x * kAddPerBlock, hi = min(B, lo + kAddPerBlock);
@@ -3458,33 +3463,81 @@ __global__ void k_zero_u32(uint32_t* v, int n){
     if(i < n) v[i] = 0u;
 }
 
-// Candidate capacity check of a batch whose candidate arrays were sized before its
-// candidates were counted (cap < 2^32): from the batch's pair count in 64 bits at
-// status[6..7], status[0] = 1 when the batch has more than `cap`, status[1] = how many
-// it has (saturated at 2^32 - 1).
-__global__ void k_cap_status(uint64_t cap, uint32_t* __restrict__ status){
-    if(blockIdx.x == 0 && threadIdx.x == 0){
-        const uint64_t t = *reinterpret_cast<const unsigned long long*>(status + 6);
-        status[0] = t > cap ? 1u : 0u;
-        status[1] = uint32_t(t < uint64_t(UINT32_MAX) ? t : uint64_t(UINT32_MAX));
+// Start of a pipelined batch: candidate counts and record sizes 0, the counts of both redo
+// lists and the status words 0 (one launch; five cost 20 us of a 260 us pass over 6,000 reads).
+__global__ void __launch_bounds__(256) k_batch_init(uint32_t* __restrict__ uniq, uint32_t* __restrict__ recBytes, int B,
+                                                    uint32_t* __restrict__ overCount, uint32_t* __restrict__ listCount,
+                                                    uint32_t* __restrict__ status){
+    FOR_GRID(i, B + 1){ uniq[i] = 0u; recBytes[i] = 0u; }
+    if(blockIdx.x == 0){
+        if(threadIdx.x < kStatusWords) status[threadIdx.x] = 0u;
+        if(threadIdx.x == 0) *overCount = 0u;
+        if(threadIdx.x == 1 && listCount) *listCount = 0u;
     }
 }
 
-// After k_cap_status: a batch over capacity gets all-zero offsets, so that the rest of its
-// kernels see no candidates and write nothing past the arrays (the batch is redone).
-__global__ void k_cap_clear(uint32_t* __restrict__ offsets, int B, const uint32_t* __restrict__ status){
+// Capacity check of a pipelined batch (status words as slotStatus lays them out): the flag and
+// the pair count, and, over capacity, offsets of 0, with which the batch's later kernels see
+// no candidates.
+__global__ void k_cap_check(uint64_t cap, uint32_t* __restrict__ offsets, int B, uint32_t* __restrict__ status){
+    const uint64_t t = *reinterpret_cast<const unsigned long long*>(status + 6);
+    const bool over = t > cap;
+    if(blockIdx.x == 0 && threadIdx.x == 0){
+        status[0] = over ? 1u : 0u;
+        status[1] = uint32_t(t < uint64_t(UINT32_MAX) ? t : uint64_t(UINT32_MAX));
+    }
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i <= B && status[0]) offsets[i] = 0u;
+    if(i <= B && over) offsets[i] = 0u;
+}
+
+// Record compaction: a wave takes 64 entries at a time (8 where that leaves the chip short of
+// waves), finds those with a record by ballot and copies them one after another, lanes over
+// bytes; wavefronts stride over the batch. Most anchors have no record: a workgroup per anchor
+// spent 212 us on 1.0M anchors with 130,000 records, where this takes about 20, and a wave per
+// candidate entry 700 us on 10.0M entries with 707,000 records, about 170. `count` (may be
+// null) receives the number of records.
+constexpr int kGatherGrid = 4096;
+constexpr uint64_t kGatherSmall = uint64_t(kGatherGrid) * (kBlock / kWave) * kWave / 8;
+template<class Size, class Src>
+__device__ __forceinline__ void copyRecords(uint64_t n, const Size* __restrict__ size, const uint64_t* __restrict__ off,
+                                              uint8_t* __restrict__ out, unsigned long long* count, Src&& src){
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint64_t waves = uint64_t(gridDim.x) * (blockDim.x / kWave);
+    const uint64_t per = n <= kGatherSmall ? 8 : kWave;
+    unsigned long long found = 0;
+    for(uint64_t base = (uint64_t(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave) * per; base < n;
+        base += waves * per){
+        const uint64_t e = base + uint64_t(lane);
+        const uint32_t nb = uint64_t(lane) < per && e < n ? uint32_t(size[e]) : 0u;
+        uint64_t mask = __ballot(nb != 0);
+        found += (unsigned long long)(__popcll(mask));
+        const uint64_t at = nb ? off[e] : 0;
+        const uint64_t from = nb ? src(e) : 0;
+        while(mask){
+            const int l = __builtin_ctzll(mask);
+            mask &= mask - 1;
+            const uint32_t bytes = uint32_t(__builtin_amdgcn_readlane(int(nb), l));
+            const uint64_t o = uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(at)), l))) |
+                               uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(at >> 32)), l))) << 32;
+            const uint64_t f = uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(from)), l))) |
+                               uint64_t(uint32_t(__builtin_amdgcn_readlane(int(uint32_t(from >> 32)), l))) << 32;
+            const uint8_t* s = reinterpret_cast<const uint8_t*>(f);
+            for(uint32_t q = lane; q < bytes; q += kWave) out[o + q] = s[q];
+        }
+    }
+    if(count && lane == 0 && found) atomicAdd(count, found);
 }
 
 __global__ void __launch_bounds__(kBlock)
-k_gather(const uint8_t* slots, int slotBytes, const uint32_t* recBytes, const uint64_t* outOff, uint8_t* out, int B){
-    const int i = blockIdx.x;
-    if(i >= B) return;
-    const uint32_t nb = recBytes[i];
-    const uint8_t* src = slots + size_t(i) * slotBytes;
-    uint8_t* dst = out + outOff[i];
-    for(uint32_t q = threadIdx.x; q < nb; q += kBlock) dst[q] = src[q];
+k_gather(const uint8_t* slots, int slotBytes, const uint32_t* recBytes, const uint64_t* outOff, uint8_t* out, int B,
+         unsigned long long* count, uint32_t* status, const int* error){
+    // a pipelined batch's record bytes and error flag, beside its other status words
+    if(status && blockIdx.x == 0 && threadIdx.x == 0){
+        *reinterpret_cast<uint64_t*>(status + 8) = outOff[B];
+        status[10] = uint32_t(*error);
+    }
+    copyRecords(uint64_t(B), recBytes, outOff, out, count,
+                  [&](uint64_t i){ return reinterpret_cast<uint64_t>(slots + i * uint64_t(slotBytes)); });
 }
 
 __global__ void k_widen(const uint32_t* in, uint64_t* out, int n){
@@ -3561,15 +3614,8 @@ __global__ void k_insertion_order(const uint32_t* __restrict__ recBytes, const u
 // One wavefront per entry: copies its record to its offset in the batch's stream.
 __global__ void __launch_bounds__(256) k_gather_entries(const uint64_t* __restrict__ size, const uint64_t* __restrict__ src,
                                                         const uint64_t* __restrict__ off, uint8_t* __restrict__ out,
-                                                        uint64_t entries){
-    const int lane = threadIdx.x & 63;
-    for(uint64_t e = (uint64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6; e < entries;
-        e += (uint64_t(gridDim.x) * blockDim.x) >> 6){
-        const uint64_t nb = size[e];
-        const uint8_t* s = reinterpret_cast<const uint8_t*>(src[e]);
-        uint8_t* d = out + off[e];
-        for(uint64_t q = lane; q < nb; q += 64) d[q] = s[q];
-    }
+                                                        uint64_t entries, unsigned long long* count){
+    copyRecords(entries, size, off, out, count, [&](uint64_t e){ return src[e]; });
 }
 
 // ---------------------------------------------------------------- host side
@@ -3990,6 +4036,13 @@ int recordSlotBytes(int maxLen){
     return ((8 + 4 + std::max(maxLen, 5 * (maxLen / 7 + 1))) + 15) / 16 * 16;
 }
 
+// Workgroups of a record gather over n entries, and the counter of a synchronized batch's records.
+dim3 gatherGrid(uint64_t n){
+    const uint64_t per = (n <= kGatherSmall ? 8 : kWave) * (kBlock / kWave);
+    return dim3(uint32_t(std::min<uint64_t>((n + per - 1) / per, kGatherGrid)));
+}
+unsigned long long* recordCounter(care_ctx* ctx){ return ctx->counters.as<unsigned long long>() + 6; }
+
 // Record compaction, device part: record sizes widened and scanned into byte offsets,
 // then the total and the error flag copied into the context's pinned host words (no host
 // synchronization; capturable). Uses the preallocated scan workspace only.
@@ -4024,31 +4077,19 @@ int recordsFinish(care_ctx* ctx, int B, int slotBytes, HostRecords& out, size_t&
     std::memcpy(&errFlag, reinterpret_cast<uint8_t*>(ctx->pinned) + 8, 4);
     if(errFlag) return ctx->fail(CARE_EINVAL, "MSA column bound exceeded");
     HIPCHECK(ctx->outBuf.ensure(std::max<uint64_t>(outBytes, 1)));
-    k_gather<<<B, kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), slotBytes, ctx->recBytes.as<uint32_t>(),
-                                   ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B);
+    unsigned long long* recs = recordCounter(ctx);
+    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(recs), 2);
+    k_gather<<<gatherGrid(B), kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), slotBytes, ctx->recBytes.as<uint32_t>(),
+                                               ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B, recs, nullptr, nullptr);
     HIPCHECK(hipGetLastError());
     const size_t old = out.size();
     HIPCHECK(out.resize(old + outBytes));
     if(outBytes) HIPCHECK(hipMemcpyAsync(out.data() + old, ctx->outBuf.p, outBytes, hipMemcpyDeviceToHost, st));
+    unsigned long long records = 0;
+    HIPCHECK(hipMemcpyAsync(&records, recs, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));
-    size_t q = old;
-    while(q < out.size()){
-        uint32_t flags;
-        memcpy(&flags, out.data() + q + 4, 4);
-        q += 8 + (flags & ((1u << 29) - 1));
-        outRecords++;
-    }
+    outRecords += size_t(records);
     return CARE_OK;
-}
-
-// Compacts the per-anchor record slots [0, B) into one buffer and appends it to `out`.
-int gatherRecords(care_ctx* ctx, int B, int slotBytes, HostRecords& out, size_t& outRecords){
-    int rc = ensureRecordScan(ctx, B);
-    if(rc != CARE_OK) return rc;
-    rc = recordsDevicePart(ctx, B);
-    if(rc != CARE_OK) return rc;
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
-    return recordsFinish(ctx, B, slotBytes, out, outRecords);
 }
 
 // Fused pass over anchors [first, first+n): one persistent kernel, then record compaction.
@@ -4216,13 +4257,17 @@ int gatherInsertionOrder(care_ctx* ctx, uint64_t b0, int B, uint32_t total, int 
     HIPCHECK(hipStreamSynchronize(st));
     if(errFlag) return ctx->fail(CARE_EINVAL, "MSA column bound exceeded in batch at %llu", (unsigned long long)b0);
     HIPCHECK(ctx->outBuf.ensure(std::max<uint64_t>(outBytes, 1)));
-    k_gather_entries<<<gridFor(entries * 64, 256), 256, 0, st>>>(
+    unsigned long long* recs = recordCounter(ctx);
+    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(recs), 2);
+    k_gather_entries<<<gatherGrid(entries), 256, 0, st>>>(
         ctx->insSize.as<uint64_t>(), ctx->insSrc.as<uint64_t>(), ctx->insOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(),
-        entries);
+        entries, recs);
     HIPCHECK(hipGetLastError());
     const size_t old = out.size();
     HIPCHECK(out.resize(old + outBytes));
     if(outBytes) HIPCHECK(hipMemcpyAsync(out.data() + old, ctx->outBuf.p, outBytes, hipMemcpyDeviceToHost, st));
+    unsigned long long records = 0;
+    HIPCHECK(hipMemcpyAsync(&records, recs, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipEventRecord(ctx->ev[4], st));
     HIPCHECK(hipStreamSynchronize(st));
     float ms = 0;
@@ -4232,13 +4277,7 @@ int gatherInsertionOrder(care_ctx* ctx, uint64_t b0, int B, uint32_t total, int 
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[3])); ctx->t.msa_ms += ms; ctx->t.msa_kernel_ms += ms;
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[3], ctx->ev[4])); ctx->t.output_ms += ms;
     ctx->t.candidates += total;
-    size_t q = old;
-    while(q < out.size()){
-        uint32_t flags;
-        memcpy(&flags, out.data() + q + 4, 4);
-        q += 8 + (flags & ((1u << 29) - 1));
-        outRecords++;
-    }
+    outRecords += size_t(records);
     return CARE_OK;
 }
 
@@ -4313,8 +4352,8 @@ hipError_t launchAlignLanes(const AlignParams& ap, int grid, int wm, hipStream_t
 }
 
 // The alignment kernel of a staged batch: the seeded kernel (seeded alignment), the matrix
-// kernel followed by the scan of the anchors it listed, the lane-per-candidate kernel
-// (wm > 0), or the wavefront-per-pair kernel over `total` pairs.
+// kernel followed by the scan of the anchors it listed (*ap.listCount is 0 before), the
+// lane-per-candidate kernel (wm > 0), or the wavefront-per-pair kernel over `total` pairs.
 hipError_t launchAlign(const care_ctx* ctx, const AlignParams& ap, int B, uint32_t total, int wm, hipStream_t st){
     if(ctx->o.seeded_alignment){
         switch(alignLaneWords(ctx->W)){
@@ -4328,7 +4367,6 @@ hipError_t launchAlign(const care_ctx* ctx, const AlignParams& ap, int B, uint32
         return hipGetLastError();
     }
     if(matrixAlign(ctx)){
-        k_zero_u32<<<1, 64, 0, st>>>(ap.listCount, 1);
         const size_t lds = size_t(matrixLds(ctx->W).bytes);
         switch((ctx->W + 1) / 2){
             case 0: case 1: k_align_matrix<1><<<B, kWave, lds, st>>>(ap); break;
@@ -4428,7 +4466,7 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     // the batch's candidate pairs in 64 bits: list offsets and indices are 32-bit
     unsigned long long* pairs64 = ctx->counters.as<unsigned long long>() + 5;
     k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(pairs64), 2);
-    k_add_gathered<<<(B + kAddPerBlock - 1) / kAddPerBlock, kBlock, 0, st>>>(ctx->uniq.as<uint32_t>(), B, pairs64);
+    k_add_gathered<<<(B + kAddPerBlock - 1) / kAddPerBlock, kBlock, 0, st>>>(ctx->uniq.as<uint32_t>(), B, pairs64, nullptr, nullptr);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(ctx->ev[5], st));
     size_t tb = 0;
@@ -4454,8 +4492,8 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
         return runBatch(ctx, b0 + uint64_t(B1), B - B1, out, outRecords);
     }
     // the batch's gathered bucket values into the pass statistic (once the batch is kept)
-    k_add_gathered<<<(B + kAddPerBlock - 1) / kAddPerBlock, kBlock, 0, st>>>(ctx->gath.as<uint32_t>(), B,
-                                                                          ctx->counters.as<unsigned long long>());
+    k_add_gathered<<<(B + kAddPerBlock - 1) / kAddPerBlock, kBlock, 0, st>>>(
+        ctx->gath.as<uint32_t>(), B, ctx->counters.as<unsigned long long>(), nullptr, nullptr);
     HIPCHECK(hipGetLastError());
     const size_t T = std::max<size_t>(total, 1);
     HIPCHECK(ctx->ids.ensure(T * 4));
@@ -4488,6 +4526,7 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     ap.offsets = ctx->offsets.as<uint32_t>(); ap.B = B; ap.maxLen = ctx->maxLen;
     ap.order = order;
     HIPCHECK(prepareAlignList(ctx, B, ap));
+    if(ap.listCount) k_zero_u32<<<1, 64, 0, st>>>(ap.listCount, 1);
     if(total) HIPCHECK(launchAlign(ctx, ap, B, total, wm, st));
     HIPCHECK(hipEventRecord(ctx->ev[2], st));
 
@@ -4566,23 +4605,20 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     HIPCHECK(hipStreamSynchronize(st));
     if(errFlag) return ctx->fail(CARE_EINVAL, "MSA column bound exceeded in batch at %llu", (unsigned long long)b0);
     HIPCHECK(ctx->outBuf.ensure(std::max<uint64_t>(outBytes, 1)));
-    k_gather<<<B, kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), slotBytes, ctx->recBytes.as<uint32_t>(),
-                                   ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B);
+    unsigned long long* recs = recordCounter(ctx);
+    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(recs), 2);
+    k_gather<<<gatherGrid(B), kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), slotBytes, ctx->recBytes.as<uint32_t>(),
+                                               ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B, recs, nullptr, nullptr);
     HIPCHECK(hipGetLastError());
     const size_t old = out.size();
     HIPCHECK(out.resize(old + outBytes));
     if(outBytes) HIPCHECK(hipMemcpyAsync(out.data() + old, ctx->outBuf.p, outBytes, hipMemcpyDeviceToHost, st));
+    unsigned long long records = 0;
+    HIPCHECK(hipMemcpyAsync(&records, recs, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipEventRecord(ctx->ev[4], st));
     HIPCHECK(hipStreamSynchronize(st));
 
-    // count records of this batch
-    size_t q = old;
-    while(q < out.size()){
-        uint32_t flags;
-        memcpy(&flags, out.data() + q + 4, 4);
-        q += 8 + (flags & ((1u << 29) - 1));
-        outRecords++;
-    }
+    outRecords += size_t(records);
     float ms;
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1])); ctx->t.candidates_ms += ms;
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[5])); ctx->t.cand_kernel_ms += ms;
@@ -4612,11 +4648,11 @@ struct StagedLaunch {
     size_t waveLds, candLds, msaLds;
 };
 
-// Status words of batch slot s: in `counters` at [64 + 32 s): over-capacity flag (u32),
-// candidate pairs (u32, saturated), bucket values gathered (u64), records (u64), candidate
-// pairs (u64); copied after the record bytes (u64) and the error flag (i32) to the pinned
-// words at [64 + 64 s): bytes 0, 8, then 16 on.
-uint32_t* slotStatus(care_ctx* ctx, int s){ return ctx->counters.as<uint32_t>() + 16 + 8 * s; }
+// Status words of batch slot s, in `counters` from byte 128 + 64 s and copied as they are to the
+// pinned words at [64 + 64 s): over-capacity flag (u32), candidate pairs (u32, saturated),
+// bucket values gathered (u64), records (u64), candidate pairs (u64), record bytes (u64),
+// error flag (i32).
+uint32_t* slotStatus(care_ctx* ctx, int s){ return ctx->counters.as<uint32_t>() + 32 + 16 * s; }
 uint8_t* slotPinned(care_ctx* ctx, int s){ return reinterpret_cast<uint8_t*>(ctx->pinned) + 64 + 64 * s; }
 
 // The device work of one pipelined batch, after its processing order (batchOrder).
@@ -4630,20 +4666,17 @@ hipError_t enqueueStaged(care_ctx* ctx, const StagedLaunch& L, bool events){
 #define ENQ(launch) do { launch; e = hipGetLastError(); if(e != hipSuccess) return e; } while(0)
 #define ENQE(expr) do { e = (expr); if(e != hipSuccess) return e; } while(0)
     uint32_t* overCount = reinterpret_cast<uint32_t*>(ctx->candOver.as<uint8_t>() + size_t(B) * 4);
-    ENQ((k_fill_u32<<<dim3(uint32_t((B + 1 + 255) / 256)), 256, 0, st>>>(L.cp.uniq, uint64_t(B + 1), 0u)));
-    ENQ((k_zero_u32<<<1, 64, 0, st>>>(overCount, 1)));
-    ENQ((k_zero_u32<<<1, 64, 0, st>>>(status, 8)));
+    ENQ((k_batch_init<<<gridFor(uint64_t(B) + 1, 256), 256, 0, st>>>(L.cp.uniq, ctx->recBytes.as<uint32_t>(), B, overCount,
+                                                                     L.ap.listCount, status)));
     ENQ((k_candidates_wave<<<B, kWave, L.waveLds, st>>>(L.cp, ctx->candOver.as<uint32_t>(), overCount)));
     ENQ((k_candidates_over<<<std::min(B, 4096), kBlock, L.candLds, st>>>(L.cp, ctx->candOver.as<uint32_t>(), overCount)));
-    ENQ((k_add_gathered<<<(B + kAddPerBlock - 1) / kAddPerBlock, kBlock, 0, st>>>(
-        ctx->gath.as<uint32_t>(), B, reinterpret_cast<unsigned long long*>(status + 2))));
-    ENQ((k_add_gathered<<<(B + kAddPerBlock - 1) / kAddPerBlock, kBlock, 0, st>>>(
-        L.cp.uniq, B, reinterpret_cast<unsigned long long*>(status + 6))));
+    ENQ((k_add_gathered<<<dim3(uint32_t((B + kAddPerBlock - 1) / kAddPerBlock), 2), kBlock, 0, st>>>(
+        ctx->gath.as<uint32_t>(), B, reinterpret_cast<unsigned long long*>(status + 2),
+        L.cp.uniq, reinterpret_cast<unsigned long long*>(status + 6))));
     if(events) ENQE(hipEventRecord(ev[5], st));
     size_t tb = ctx->scanTmp.bytes;
     ENQE(hipcub::DeviceScan::ExclusiveSum(ctx->scanTmp.p, tb, ctx->uniq.as<uint32_t>(), ctx->offsets.as<uint32_t>(), B + 1, st));
-    ENQ((k_cap_status<<<1, 64, 0, st>>>(L.cap, status)));
-    ENQ((k_cap_clear<<<(B + 1 + 255) / 256, 256, 0, st>>>(ctx->offsets.as<uint32_t>(), B, status)));
+    ENQ((k_cap_check<<<(B + 1 + 255) / 256, 256, 0, st>>>(L.cap, ctx->offsets.as<uint32_t>(), B, status)));
     ENQ((k_compact<<<(B + kBlock / kWave - 1) / (kBlock / kWave), kBlock, 0, st>>>(
         ctx->raw.as<uint32_t>(), L.capPerAnchor, ctx->offsets.as<uint32_t>(), B, ctx->ids.as<uint32_t>(), nullptr)));
     if(ctx->o.paired){
@@ -4654,7 +4687,6 @@ hipError_t enqueueStaged(care_ctx* ctx, const StagedLaunch& L, bool events){
     if(events) ENQE(hipEventRecord(ev[1], st));
     ENQE(launchAlign(ctx, L.ap, B, 0, L.wm, st));
     if(events) ENQE(hipEventRecord(ev[2], st));
-    ENQ((k_fill_u32<<<dim3(uint32_t((B + 1 + 255) / 256)), 256, 0, st>>>(ctx->recBytes.as<uint32_t>(), uint64_t(B + 1), 0u)));
     if(L.kc > 0){
         ENQE(launchWaveMsa(L.mp, B, L.kc, L.wholeMsa != 0, L.q != 0, L.msaLds, st));
     }else{
@@ -4665,12 +4697,11 @@ hipError_t enqueueStaged(care_ctx* ctx, const StagedLaunch& L, bool events){
                                                             reinterpret_cast<unsigned long long*>(status + 4))));
     tb = ctx->scanTmp.bytes;
     ENQE(hipcub::DeviceScan::ExclusiveSum(ctx->scanTmp.p, tb, ctx->recOff64.as<uint64_t>(), ctx->recOff.as<uint64_t>(), B + 1, st));
-    ENQ((k_gather<<<B, kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), L.slotBytes, ctx->recBytes.as<uint32_t>(),
-                                        ctx->recOff.as<uint64_t>(), ctx->pipeOut[L.slot].as<uint8_t>(), B)));
+    ENQ((k_gather<<<gatherGrid(B), kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), L.slotBytes, ctx->recBytes.as<uint32_t>(),
+                                                    ctx->recOff.as<uint64_t>(), ctx->pipeOut[L.slot].as<uint8_t>(), B, nullptr,
+                                                    status, ctx->counters.as<int>() + 2)));
     uint8_t* pw = slotPinned(ctx, L.slot);
-    ENQE(hipMemcpyAsync(pw, ctx->recOff.as<uint64_t>() + B, 8, hipMemcpyDeviceToHost, st));
-    ENQE(hipMemcpyAsync(pw + 8, ctx->counters.as<int>() + 2, 4, hipMemcpyDeviceToHost, st));
-    ENQE(hipMemcpyAsync(pw + 16, status, 32, hipMemcpyDeviceToHost, st));
+    ENQE(hipMemcpyAsync(pw, status, kStatusWords * 4, hipMemcpyDeviceToHost, st));
 #undef ENQ
 #undef ENQE
     return hipSuccess;
@@ -4834,12 +4865,12 @@ int finishStaged(care_ctx* ctx, uint64_t b0, int B, int slot, HostRecords& out, 
     uint64_t outBytes = 0, gath = 0, recs = 0;
     int errFlag = 0;
     uint32_t over = 0, total = 0;
-    std::memcpy(&outBytes, pw, 8);
-    std::memcpy(&errFlag, pw + 8, 4);
-    std::memcpy(&over, pw + 16, 4);
-    std::memcpy(&total, pw + 20, 4);
-    std::memcpy(&gath, pw + 24, 8);
-    std::memcpy(&recs, pw + 32, 8);
+    std::memcpy(&over, pw, 4);
+    std::memcpy(&total, pw + 4, 4);
+    std::memcpy(&gath, pw + 8, 8);
+    std::memcpy(&recs, pw + 16, 8);
+    std::memcpy(&outBytes, pw + 32, 8);
+    std::memcpy(&errFlag, pw + 40, 4);
     if(errFlag) return ctx->fail(CARE_EINVAL, "MSA column bound exceeded in batch at %llu", (unsigned long long)b0);
     ctx->candPerAnchor = std::max(ctx->candPerAnchor, double(total) / double(std::max(B, 1)));
     float ms = 0;
@@ -6605,7 +6636,7 @@ static int care_hip_correct_body(care_ctx* ctx, uint64_t first, uint64_t n, size
     ctx->t = care_timings{};
     ctx->records.clear();
     ctx->numRecords = 0;
-    HIPCHECK(ctx->counters.ensure(128));
+    HIPCHECK(ctx->counters.ensure(256));
     HIPCHECK(hipMemsetAsync(ctx->counters.p, 0, 128, ctx->stream));
     int B = ctx->o.batch_size > 0 ? ctx->o.batch_size : 0;
     if(B <= 0){
@@ -6675,8 +6706,9 @@ static int care_hip_correct_body(care_ctx* ctx, uint64_t first, uint64_t n, size
             b0 = e;
         }
     }
+    // (pipelined batches report through their status words; redone ones count as the others do)
     unsigned long long cnt[4] = {0, 0, 0, 0};
-    HIPCHECK(hipMemcpy(cnt, ctx->counters.p, 32, hipMemcpyDeviceToHost));
+    if(!pipelined || ctx->t.batches_redone) HIPCHECK(hipMemcpy(cnt, ctx->counters.p, 32, hipMemcpyDeviceToHost));
     const unsigned long long gathered = cnt[0] + pipeGathered;
     if(fused) ctx->t.candidates = cnt[3];
     const auto t1 = std::chrono::steady_clock::now();
