@@ -25,17 +25,17 @@
 // about the same for any sequence: an exact count costs some 4 instructions per shift, the
 // scan of every shift some 150 per candidate.
 //
-// Measured (k_align, MI355X): 1.0M x 150 bases 12.15 -> 4.8 ms against the lane scan, 1.03M
-// reads of 100..250 bases 28.8 -> 9.1 ms, 60,000 of 360..450 bases 7.4 -> 1.2 ms against the
-// wavefront per pair. At 150 bases: 3.0k vector instructions per anchor (1.1 per clock and
-// CU at 5.9 waves per SIMD), matrix cores busy 16% of the time, of 18 products per block;
-// bound by vector issue and by the latency of its LDS and accumulator reads.
+// Measured (MI355X): 1.0M x 150 bases 12.15 -> 4.6 ms against the lane scan, 1.03M reads of
+// 100..250 bases 28.8 -> 8.5 ms, 60,000 of 360..450 bases 7.4 -> 1.2 ms against the wavefront
+// per pair. At 150 bases: 2.9k vector and 1.5k scalar instructions per anchor (1.1 and 0.6
+// per clock and CU at 5.9 waves per SIMD), matrix cores busy a fifth of the time; bound by
+// instruction issue and by the latency of its LDS and accumulator reads.
 //
 // Position order inside a 64-deep step is free as long as both operands share it: dword i
 // of a lane's 32 positions holds positions 4n + i in nibbles n, so a nibble dword is one
 // shift and one and-or from a plane word, and the anchor's dword i at bit offset o is its
 // dword 0 at offset o + i: one LDS dword per bit offset feeds the whole Toeplitz matrix
-// (a lane reads four consecutive ones; 4.4 KB of LDS per wave at 150 bases, where 16-byte
+// (a lane reads four consecutive ones; 4.7 KB of LDS per wave at 150 bases, where 16-byte
 // fragments took 7.9 KB and held the kernel at 4.3 waves per SIMD).
 
 typedef int MatrixFrag __attribute__((ext_vector_type(8)));
@@ -57,7 +57,7 @@ __host__ __device__ inline MatrixLds matrixLds(int W){
     MatrixLds l;
     const int pairs = 2 * 2 * (W + 6);              // uint2 per word index -4..W+1, two planes
     l.frag = (pairs + 3) & ~3;
-    l.rows = l.frag + (W + 4) * 32 + 4;             // bit offsets from word -3 on
+    l.rows = l.frag + (W + 6) * 32 + 4;             // bit offsets from word -4 on
     l.rowStride = 4 * W + 4;                        // 16 bytes of padding against bank conflicts
     l.queue = l.rows + kMatrixCands * l.rowStride;
     l.keys = l.queue + kMatrixQueue;
@@ -76,6 +76,15 @@ __device__ __forceinline__ int signNibbles(uint32_t v, uint32_t m, int i){
 // NaN quieting, which costs fmaxf a second instruction per operand)
 __device__ __forceinline__ float maxNegative(float x, float y){
     return __uint_as_float(min(__float_as_uint(x), __float_as_uint(y)));
+}
+
+// Least and largest value over the 16 lanes of a row (DPP: neighbours, pairs, mirrored halves).
+__device__ __forceinline__ void rowMinMax(int& lo, int& hi){
+#define ROW_STEP(ctrl) \
+    lo = min(lo, __builtin_amdgcn_update_dpp(lo, lo, ctrl, 0xf, 0xf, false)); \
+    hi = max(hi, __builtin_amdgcn_update_dpp(hi, hi, ctrl, 0xf, 0xf, false));
+    ROW_STEP(0xB1) ROW_STEP(0x4E) ROW_STEP(0x141) ROW_STEP(0x140)     // quad_perm 1,0,3,2 / 2,3,0,1, half mirror, mirror
+#undef ROW_STEP
 }
 
 template<int KB>
@@ -121,11 +130,12 @@ k_align_matrix(AlignParams p){
     const int sAlign = sTop + 1;                        // blocks start at sAlign - 32 * k
     const int delta = sAlign & 31;
     const int Wa = (La + 31) >> 5;
-    // nibble dword 0 of the 32 anchor positions from bit offset 32 * -3 + delta + q
-    for(int q = lane; q < (W + 4) * 32 + 4; q += kWave){
-        const int o = q - 96 + delta;
-        const uint2 pr = aPair[pairs + min(o >> 5, W + 1) + 4];
-        const uint32_t v = uint32_t((((uint64_t(pr.y) << 32) | pr.x) << (o & 31)) >> 32);
+    // nibble dword 0 of the 32 anchor positions from bit offset 32 * -4 + delta + q (all zero in
+    // words -4, -3 of the first half's and W, W + 1 of the second half's rows)
+    for(int q = lane; q < (W + 6) * 32 + 4; q += kWave){
+        const int o = q - 128 + delta;
+        const uint2 pr = aPair[pairs + min(max(((o + 31) >> 5) + 3, 0), pairs - 1)];
+        const uint32_t v = __builtin_amdgcn_alignbit(pr.y, pr.x, uint32_t(-o) & 31u);
         const uint32_t m = overlapMask(La - o) & ~overlapMask(-o);
         frag[q] = uint32_t(signNibbles(v & m, m, 0));
     }
@@ -183,28 +193,31 @@ k_align_matrix(AlignParams p){
             const int ci = b * kMatrixCands + (lane & 15);
             const bool cvalid = ci < cn;
             const int lc = cvalid ? lens[ci] : 0;
-            // candidate fragments of this lane's column
+            // longest and shortest candidate of the block (wave-uniform)
+            int lcMax = lc, lcMin = cvalid ? lc : INT_MAX;
+            rowMinMax(lcMin, lcMax);
+            lcMax = __builtin_amdgcn_readfirstlane(lcMax);
+            lcMin = __builtin_amdgcn_readfirstlane(lcMin);
+            // candidate fragments of this lane's column (no masks where every candidate of the block
+            // covers the step's positions)
             MatrixFrag B[KB];
             {
                 const uint32_t* lo = rows + (lane & 15) * L.rowStride + (orient ? 3 * W : W);
                 #pragma unroll
                 for(int kb = 0; kb < KB; kb++){
                     const int w = 2 * kb + half;
-                    const uint32_t m = cvalid ? overlapMask(lc - 32 * w) : 0u;
-                    const uint32_t v = m && w < W ? lo[w] & m : 0u;
-                    B[kb] = MatrixFrag{signNibbles(v, m, 0), signNibbles(v, m, 1), signNibbles(v, m, 2),
-                                       signNibbles(v, m, 3), 0, 0, 0, 0};
+                    if(lcMin >= 64 * (kb + 1)){
+                        const uint32_t v = lo[w];
+                        B[kb] = MatrixFrag{signNibbles(v, ~0u, 0), signNibbles(v, ~0u, 1), signNibbles(v, ~0u, 2),
+                                           signNibbles(v, ~0u, 3), 0, 0, 0, 0};
+                    }else{
+                        const uint32_t m = cvalid ? overlapMask(lc - 32 * w) : 0u;
+                        const uint32_t v = m && w < W ? lo[w] & m : 0u;
+                        B[kb] = MatrixFrag{signNibbles(v, m, 0), signNibbles(v, m, 1), signNibbles(v, m, 2),
+                                           signNibbles(v, m, 3), 0, 0, 0, 0};
+                    }
                 }
             }
-            // longest and shortest candidate of the block (wave-uniform)
-            int lcMax = lc, lcMin = cvalid ? lc : INT_MAX;
-            #pragma unroll
-            for(int o = 1; o < 16; o <<= 1){
-                lcMax = max(lcMax, __shfl_xor(lcMax, o));
-                lcMin = min(lcMin, __shfl_xor(lcMin, o));
-            }
-            lcMax = __builtin_amdgcn_readfirstlane(lcMax);
-            lcMin = __builtin_amdgcn_readfirstlane(lcMin);
             const int nkb = (lcMax + 63) >> 6;
             const int lastB = max(lc - mo, 0);          // -lastB: most negative shift of this lane's candidate
             const int lastBMin = max(lcMin - mo, 0);
@@ -227,14 +240,14 @@ k_align_matrix(AlignParams p){
                         const uint32_t* crow = rows + ec * L.rowStride + eo * 2 * W;
                         const int cbeg = max(-s, 0), cend = min(el, La - s);
                         for(int j = lane & 1; 32 * j < cend; j += 2){
-                            const int lo = min(max(cbeg - 32 * j, 0), 32), hi = min(max(cend - 32 * j, 0), 32);
-                            if(hi > lo){
-                                const uint32_t mask = uint32_t((0xFFFFFFFFull >> lo) & ~(0xFFFFFFFFull >> hi));
+                            const int lo = cbeg - 32 * j, hi = cend - 32 * j;   // hi > 0
+                            if(lo < 32){
+                                const uint32_t mask = (0xFFFFFFFFu >> max(lo, 0)) & (hi >= 32 ? ~0u : ~(0xFFFFFFFFu >> (hi & 31)));
                                 const int o = 32 * j + s;               // in (-32, La)
-                                const int r = o & 31;
-                                const uint2 vh = aPair[(o >> 5) + 4], vl = aPair[pairs + (o >> 5) + 4];
-                                const uint32_t ah = uint32_t((((uint64_t(vh.y) << 32) | vh.x) << r) >> 32);
-                                const uint32_t al = uint32_t((((uint64_t(vl.y) << 32) | vl.x) << r) >> 32);
+                                const int at = ((o + 31) >> 5) + 3;     // words above and below the window's end
+                                const uint2 vh = aPair[at], vl = aPair[pairs + at];
+                                const uint32_t ah = __builtin_amdgcn_alignbit(vh.y, vh.x, uint32_t(-o) & 31u);
+                                const uint32_t al = __builtin_amdgcn_alignbit(vl.y, vl.x, uint32_t(-o) & 31u);
                                 mis += __popc(((ah ^ crow[j]) | (al ^ crow[W + j])) & mask);
                             }
                         }
@@ -283,8 +296,12 @@ k_align_matrix(AlignParams p){
                     #pragma unroll
                     for(int kb = 0; kb < KB; kb++){
                         const int x = xb + 2 * kb;      // word offset of this depth step's first half
-                        if(kb < nkb && x >= -3 && x < Wa){
-                            const uint32_t* f = frag + (x + half + 3) * 32 + col;
+                        // up to 3 steps run whether the anchor reaches them or not (x held in
+                        // its zero words): a test and a branch per step cost more than the
+                        // product, the scalar unit being nearly as busy as the vector unit
+                        // (150 bases: 4.8 -> 4.6 ms; 4 steps on 100..250 bases: 8.5 -> 8.6 ms)
+                        if(KB <= 3 || (kb < nkb && x >= -3 && x < Wa)){
+                            const uint32_t* f = frag + (min(max(x, -4), W) + half + 4) * 32 + col;
                             const MatrixFrag A = {int(f[0]), int(f[1]), int(f[2]), int(f[3]), 0, 0, 0, 0};
                             acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B[kb], acc, 4, 4, 0, 0, 0, 0);
                         }
