@@ -2265,71 +2265,18 @@ __device__ __forceinline__ int countOf(const WaveMsa<KC>& m, int k, int b){
     return int(uint32_t(m.cnt[k] >> (16 * b)) & 0xFFFFu);
 }
 
-// MSA of the anchor and the first nk working candidates (src/msa.cpp:9-173), one wave:
-// every lane adds the anchor then the candidates, in list order, to the columns it owns.
-// AO (anchor columns only): slot column c is anchor position c, and only the columns
-// under the anchor are built; every later step of the plain correction (refinement,
-// properties, decision, features) reads no other column. Otherwise slot column c is MSA
-// column c (anchor position c - ab), all ncol columns. QM: 0 = no quality scores,
-// 1 = quality scores, 2 = as p.useQ says at run time.
-template<int KC, bool AO, int QM>
-__device__ __forceinline__ bool buildMsaWave(const MsaParams& p, const AnchorLists& lst, uint64_t a, int La,
-                                             const uint32_t* arow, int beg, int nk,
-                             WaveMsa<KC>& m, const MsaTile& t, int lane, bool inLanes = false,
-                             const LaneCand& lc = LaneCand{}){
-    // inLanes (wave-uniform, nk <= 64): lane i holds candidate i of the working list, which
-    // the list in memory holds as well
-    int lo = 0, hi = La;
-    for(int j = lane; j < nk; j += kWave){
-        const int s = inLanes ? lc.shift : lst.kShift[beg + j];
-        lo = min(lo, s);
-        hi = max(hi, s + (inLanes ? lc.len : lst.kLen[beg + j]));
-    }
-    lo = waveReduce(lo, OpMin(), INT_MAX);
-    hi = waveReduce(hi, OpMax(), INT_MIN);
-    const int ncol = hi - lo;
-    const int ab = max(-lo, 0);
-    if((AO ? La : ncol) > KC * kWave || ncol > p.maxCols) return false;
-    m.ncol = ncol;
-    m.ab = ab;
-    m.abase = 0;
-    m.isAnchor = 0;
-    const int off = AO ? 0 : ab;       // slot column of anchor position 0
+// Adds (SUB: subtracts) the candidates of one chunk, held in lanes 0..cn-1, to the columns in list
+// order: they are staged into LDS a tile at a time, and every lane takes the bases at the
+// columns it owns.
+template<int KC, bool AO, int QM, bool SUB>
+__device__ __forceinline__ void addCandidates(const MsaParams& p, WaveMsa<KC>& m, const MsaTile& t, const LaneCand& c, int cn,
+                                              int La, int off, int lane){
     const bool useQ = QM == 2 ? p.useQ != 0 : QM == 1;
-    const uint8_t* aq = useQ ? p.qual + p.qdpitch * a : nullptr;
-    #pragma unroll
-    for(int k = 0; k < KC; k++){
-        #pragma unroll
-        for(int b = 0; b < 4; b++) m.w[k][b] = 0.0f;
-        m.cnt[k] = 0;
-        const int pa = lane + kWave * k - off;
-        if(pa >= 0 && pa < La){
-            const int b = baseAt(arow, pa);
-            const float x = 1.0f * (useQ ? t.qw[aq[pa]] : 1.0f);
-            m.w[k][0] = b == 0 ? x : 0.0f;
-            m.w[k][1] = b == 1 ? x : 0.0f;
-            m.w[k][2] = b == 2 ? x : 0.0f;
-            m.w[k][3] = b == 3 ? x : 0.0f;
-            m.cnt[k] = uint64_t(1) << (16 * b);
-            m.abase |= uint32_t(b) << (2 * k);
-            m.isAnchor |= 1u << k;
-        }
-    }
     const int RS = 2 * p.W;                  // tile row stride in words
     const int T = p.tile;
     const int qs = qStride(p.maxLen);
     const int qrc = rcQualityOffset(p);
-    // chunks of 64 candidates: lane i holds candidate i of the chunk
-    for(int cb = 0; cb < nk; cb += kWave){
-    LaneCand c = lc;
-    if(!inLanes){
-        c = LaneCand{};
-        const int d = beg + cb + lane;
-        if(cb + lane < nk){
-            c.id = lst.kId[d]; c.shift = lst.kShift[d]; c.len = lst.kLen[d]; c.orient = lst.kOrient[d]; c.w = lst.kW[d];
-        }
-    }
-    const int cn = min(kWave, nk - cb);
+    const float scaled = c.w * (SUB ? -0x1p24f : 0x1p24f);
     for(int tb = 0; tb < cn; tb += T){
         const int tn = min(T, cn - tb);
         __syncthreads();
@@ -2341,7 +2288,7 @@ __device__ __forceinline__ bool buildMsaWave(const MsaParams& p, const AnchorLis
         for(int j = 0; j < tn; j++){
             const int cs = off + __builtin_amdgcn_readlane(c.shift, tb + j);   // slot column of its first base
             const int ln = __builtin_amdgcn_readlane(c.len, tb + j);
-            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c.w * 0x1p24f), tb + j));
+            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(scaled), tb + j));
             const bool rc = __builtin_amdgcn_readlane(mRc, tb + j) != 0;
             // slots holding its columns (AO: those under the anchor; lanes past the anchor
             // end add to columns that are never read)
@@ -2396,13 +2343,16 @@ __device__ __forceinline__ bool buildMsaWave(const MsaParams& p, const AnchorLis
                     const Half4 hot = __builtin_bit_cast(Half4, inc);
                     #pragma unroll
                     for(int q = 0; q < 4; q++) m.w[k][q] = __builtin_fmaf(x[g], float(hot[q]), m.w[k][q]);
-                    m.cnt[k] += inc;
+                    m.cnt[k] += SUB ? 0 - inc : inc;
                 }
             }
         }
     }
-    }
-    // consensus and support (src/msa.cpp:135-157)
+}
+
+// Consensus and support of every slot (src/msa.cpp:135-157).
+template<int KC, bool AO>
+__device__ __forceinline__ void finishColumns(WaveMsa<KC>& m, int lane){
     m.cons = 0;
     #pragma unroll
     for(int k = 0; k < KC; k++){
@@ -2413,9 +2363,74 @@ __device__ __forceinline__ bool buildMsaWave(const MsaParams& p, const AnchorLis
         if(m.w[k][3] > cw){ cb = 3; cw = m.w[k][3]; }
         m.cons |= uint32_t(cb) << (2 * k);
         const float colW = m.w[k][0] + m.w[k][1] + m.w[k][2] + m.w[k][3];
-        const bool inMsa = AO ? ((m.isAnchor >> k) & 1u) != 0 : lane + kWave * k < ncol;
+        const bool inMsa = AO ? ((m.isAnchor >> k) & 1u) != 0 : lane + kWave * k < m.ncol;
         m.sup[k] = inMsa ? cw / colW : 0.0f;
     }
+}
+
+// MSA of the anchor and the first nk working candidates (src/msa.cpp:9-173), one wave:
+// every lane adds the anchor then the candidates, in list order, to the columns it owns.
+// AO (anchor columns only): slot column c is anchor position c, and only the columns
+// under the anchor are built; every later step of the plain correction (refinement,
+// properties, decision, features) reads no other column. Otherwise slot column c is MSA
+// column c (anchor position c - ab), all ncol columns. QM: 0 = no quality scores,
+// 1 = quality scores, 2 = as p.useQ says at run time.
+template<int KC, bool AO, int QM>
+__device__ __forceinline__ bool buildMsaWave(const MsaParams& p, const AnchorLists& lst, uint64_t a, int La,
+                                             const uint32_t* arow, int beg, int nk,
+                             WaveMsa<KC>& m, const MsaTile& t, int lane, bool inLanes = false,
+                             const LaneCand& lc = LaneCand{}){
+    // inLanes (wave-uniform, nk <= 64): lane i holds candidate i of the working list, which
+    // the list in memory holds as well
+    int lo = 0, hi = La;
+    for(int j = lane; j < nk; j += kWave){
+        const int s = inLanes ? lc.shift : lst.kShift[beg + j];
+        lo = min(lo, s);
+        hi = max(hi, s + (inLanes ? lc.len : lst.kLen[beg + j]));
+    }
+    lo = waveReduce(lo, OpMin(), INT_MAX);
+    hi = waveReduce(hi, OpMax(), INT_MIN);
+    const int ncol = hi - lo;
+    const int ab = max(-lo, 0);
+    if((AO ? La : ncol) > KC * kWave || ncol > p.maxCols) return false;
+    m.ncol = ncol;
+    m.ab = ab;
+    m.abase = 0;
+    m.isAnchor = 0;
+    const int off = AO ? 0 : ab;       // slot column of anchor position 0
+    const bool useQ = QM == 2 ? p.useQ != 0 : QM == 1;
+    const uint8_t* aq = useQ ? p.qual + p.qdpitch * a : nullptr;
+    #pragma unroll
+    for(int k = 0; k < KC; k++){
+        #pragma unroll
+        for(int b = 0; b < 4; b++) m.w[k][b] = 0.0f;
+        m.cnt[k] = 0;
+        const int pa = lane + kWave * k - off;
+        if(pa >= 0 && pa < La){
+            const int b = baseAt(arow, pa);
+            const float x = 1.0f * (useQ ? t.qw[aq[pa]] : 1.0f);
+            m.w[k][0] = b == 0 ? x : 0.0f;
+            m.w[k][1] = b == 1 ? x : 0.0f;
+            m.w[k][2] = b == 2 ? x : 0.0f;
+            m.w[k][3] = b == 3 ? x : 0.0f;
+            m.cnt[k] = uint64_t(1) << (16 * b);
+            m.abase |= uint32_t(b) << (2 * k);
+            m.isAnchor |= 1u << k;
+        }
+    }
+    // chunks of 64 candidates: lane i holds candidate i of the chunk
+    for(int cb = 0; cb < nk; cb += kWave){
+        LaneCand c = lc;
+        if(!inLanes){
+            c = LaneCand{};
+            const int d = beg + cb + lane;
+            if(cb + lane < nk){
+                c.id = lst.kId[d]; c.shift = lst.kShift[d]; c.len = lst.kLen[d]; c.orient = lst.kOrient[d]; c.w = lst.kW[d];
+            }
+        }
+        addCandidates<KC, AO, QM, false>(p, m, t, c, min(kWave, nk - cb), La, off, lane);
+    }
+    finishColumns<KC, AO>(m, lane);
     return true;
 }
 
@@ -2734,6 +2749,53 @@ __device__ __forceinline__ void writeRecord(const MsaParams& p, uint64_t a, int 
     }
 }
 
+// Whether every decision about the anchor comes out the same for any column weights within
+// weightError of m's (counts are exact): the thresholds on the supports, and in an anchor that
+// misses them the support test of the columns that differ from the consensus. The learned
+// seam and the feature output want exact features for such columns.
+template<int KC>
+__device__ __forceinline__ bool decidedWithin(const MsaParams& p, const WaveMsa<KC>& m, float weightError, int La){
+    float least = 2.0f, leastHi = 2.0f;
+    int sum = 0, off = 0, mincov = INT_MAX;
+    bool differs = false, near = false;
+    #pragma unroll
+    for(int k = 0; k < KC; k++){
+        if(!((m.isAnchor >> k) & 1u)) continue;
+        const float colW = m.w[k][0] + m.w[k][1] + m.w[k][2] + m.w[k][3];
+        const float e = fminf(6.0f * weightError / fmaxf(colW, 1e-3f) + 1e-6f, 1.0f);
+        const float s = m.sup[k];
+        least = fminf(least, s - e);
+        leastHi = fminf(leastHi, s + e);
+        sum += int(s * 1048576.0f);
+        off += int(e * 1048576.0f) + 2;
+        mincov = min(mincov, countOf(m, k, 0) + countOf(m, k, 1) + countOf(m, k, 2) + countOf(m, k, 3));
+        const int ob = int((m.abase >> (2 * k)) & 3u);
+        if(ob != int((m.cons >> (2 * k)) & 3u)){
+            differs = true;
+            near |= countOf(m, k, ob) <= 2 && fabsf(s - 0.90f) <= e;
+        }
+    }
+    // (supports are at most 1 and La at most 1024: the sums fit 31 bits)
+    const float scale = 1.0f / (1048576.0f * float(La));
+    const float avg = float(waveReduce(sum, OpSum(), 0)) * scale;
+    const float avgOff = float(waveReduce(off, OpSum(), 0)) * scale + 2e-4f;
+    // floats ordered as integers after moving them to [1, 4)
+    const float lo = __int_as_float(waveReduce(__float_as_int(fmaxf(least, -0.5f) + 1.5f), OpMin(), INT_MAX)) - 1.5f - 1e-6f;
+    const float hi = __int_as_float(waveReduce(__float_as_int(fmaxf(leastHi, -0.5f) + 1.5f), OpMin(), INT_MAX)) - 1.5f + 1e-6f;
+    mincov = waveReduce(mincov, OpMin(), INT_MAX);
+    const bool covered = fgeq(float(mincov), p.minCovThr);
+    const bool differing = __ballot(differs) != 0, nearing = __ballot(near) != 0;
+    const bool exactFeatures = p.seamMode != 0 || p.featOut != nullptr;
+    const bool goodSure = covered && avg - avgOff >= p.avgThr && lo >= p.minThr;
+    const bool goodMaybe = covered && avg + avgOff >= p.avgThr - 2e-5f && hi >= p.minThr - 2e-5f;
+    if(goodSure != goodMaybe) return false;
+    if(!goodSure) return !nearing && !(exactFeatures && differing);
+    const bool hqSure = avg - avgOff >= p.hqAvgT && lo >= p.hqMinT;
+    const bool hqMaybe = avg + avgOff >= p.hqAvgT - 2e-5f && hi >= p.hqMinT - 2e-5f;
+    if(hqSure != hqMaybe) return false;
+    return hqSure || !(exactFeatures && differing);
+}
+
 // Filters, MSA, refinement, decision and record of anchor `a` by one wavefront
 // (include/corrector.hpp:982-1446,1639-1761; src/msa.cpp:9-453,532-734). Its candidates
 // are lst.ids/lst.best/lst.paired[beg, beg+n0); the record goes to slot `i`.
@@ -2916,6 +2978,17 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
         if(lane == 0) atomicAdd(p.error, 1);
         return;
     }
+    // Refinement rounds take the removed candidates out of the columns instead of adding up the
+    // kept ones again (60% of the stage's candidate rows were added in rounds on 1.03M reads of
+    // 100..250 bases with repeats: 8.7 -> 6.2 ms; 500,000 pairs 5.9 -> 4.7 ms). Not for the long
+    // reads' kernels, whose registers would spill. Counts stay exact; a weight then differs from the
+    // reference's sum over the kept list by at most weightError: each of at most 3 * covMax
+    // additions (the first build's, the removals, the reference's own) rounds a sum of at
+    // most covMax by half a unit in the last place. What is decided from such columns is decided
+    // with that margin, or the columns are built again (approximate = false).
+    constexpr bool kIncremental = AO && QM != 2 && KC <= 8;
+    bool approximate = false;
+    float weightError = 0.0f;
     int rounds = 0;
     for(int it = 0; it < 5; it++){
         bool mis = false;
@@ -2969,10 +3042,10 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
         for(int base = 0; base < nk; base += kWave){
             const int j = base + lane;
             bool keep = false;
-            uint32_t id = 0; int s = 0, l = 0, no = 0, ov = 0; uint8_t o = 0, pr = 0; float w = 0.0f;
+            uint32_t id = 0; int s = 0, l = 0; uint8_t o = 0; float w = 0.0f;
             if(j < nk){
-                id = lst.kId[beg + j]; s = lst.kShift[beg + j]; l = lst.kLen[beg + j]; no = lst.kNops[beg + j];
-                ov = lst.kOvl[beg + j]; o = lst.kOrient[beg + j]; pr = lst.kPaired[beg + j]; w = lst.kW[beg + j];
+                id = lst.kId[beg + j]; s = lst.kShift[beg + j]; l = lst.kLen[beg + j];
+                o = lst.kOrient[beg + j]; w = lst.kW[beg + j];
                 const int rb = m.ab + s;
                 keep = true;
                 if(col >= rb && col < rb + l){
@@ -2983,14 +3056,68 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
             const uint64_t mask = __ballot(keep);
             if(keep){
                 const int d = beg + nn + __popcll(mask & below);
-                lst.kId[d] = id; lst.kShift[d] = s; lst.kLen[d] = l; lst.kNops[d] = no; lst.kOvl[d] = ov;
-                lst.kOrient[d] = o; lst.kPaired[d] = pr; lst.kW[d] = w;
+                // (operations, overlap and pair flag are not read after the filters)
+                lst.kId[d] = id; lst.kShift[d] = s; lst.kLen[d] = l; lst.kOrient[d] = o; lst.kW[d] = w;
             }
             nn += __popcll(mask);
+            if constexpr(kIncremental){
+                // the chunk's removed candidates, moved into lanes 0.. (a permutation)
+                const bool gone = j < nk && !keep;
+                const uint64_t goneMask = __ballot(gone);
+                if(goneMask){
+                    const int ng = __popcll(goneMask);
+                    const int dl = gone ? __popcll(goneMask & below) : ng + __popcll(~goneMask & below);
+                    LaneCand g;
+                    g.id = uint32_t(__builtin_amdgcn_ds_permute(4 * dl, int(id)));
+                    g.shift = __builtin_amdgcn_ds_permute(4 * dl, s);
+                    g.len = __builtin_amdgcn_ds_permute(4 * dl, l);
+                    g.orient = __builtin_amdgcn_ds_permute(4 * dl, int(o));
+                    g.w = __int_as_float(__builtin_amdgcn_ds_permute(4 * dl, __float_as_int(w)));
+                    if(!approximate){
+                        int cov = 0;
+                        #pragma unroll
+                        for(int k = 0; k < KC; k++)
+                            cov = max(cov, countOf(m, k, 0) + countOf(m, k, 1) + countOf(m, k, 2) + countOf(m, k, 3));
+                        const float c = float(waveReduce(cov, OpMax(), 0));
+                        weightError = 3.0f * c * c * 0x1p-24f;
+                        approximate = true;
+                    }
+                    addCandidates<KC, AO, QM, true>(p, m, tile, g, ng, La, 0, lane);
+                }
+            }
         }
         nk = nn;
         rounds++;
+        if constexpr(kIncremental){
+            // bases without a candidate left weigh exactly 0; the consensus stands where it leads
+            // by more than both sums can be off
+            bool close = false;
+            #pragma unroll
+            for(int k = 0; k < KC; k++){
+                #pragma unroll
+                for(int b = 0; b < 4; b++) if(countOf(m, k, b) == 0) m.w[k][b] = 0.0f;
+                if((m.isAnchor >> k) & 1u){
+                    const float w01 = fmaxf(m.w[k][0], m.w[k][1]), v01 = fminf(m.w[k][0], m.w[k][1]);
+                    const float w23 = fmaxf(m.w[k][2], m.w[k][3]), v23 = fminf(m.w[k][2], m.w[k][3]);
+                    const float first = fmaxf(w01, w23), second = fmaxf(fminf(w01, w23), fmaxf(v01, v23));
+                    close |= second != 0.0f && first - second <= 2.0f * weightError + 1e-6f;
+                }
+            }
+            if(__ballot(close) == 0){
+                finishColumns<KC, AO>(m, lane);
+                continue;
+            }
+            approximate = false;
+        }
         if(!buildMsaWave<KC, AO, QM>(p, lst, a, La, arow, beg, nk, m, tile, lane)){
+            if(lane == 0) atomicAdd(p.error, 1);
+            return;
+        }
+    }
+    if constexpr(kIncremental){
+        if(approximate && nk > 0 &&
+           !decidedWithin<KC>(p, m, weightError, La) &&
+           !buildMsaWave<KC, AO, QM>(p, lst, a, La, arow, beg, nk, m, tile, lane)){
             if(lane == 0) atomicAdd(p.error, 1);
             return;
         }
@@ -3182,7 +3309,7 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
 
 template<int KC, bool AO, int QM>
 __global__ void __launch_bounds__(kWave)
-__attribute__((amdgpu_waves_per_eu(AO && KC <= 3 ? 6 : (AO && KC <= 4 ? 5 : (KC <= 8 ? 4 : 2)))))
+__attribute__((amdgpu_waves_per_eu(AO ? (KC <= 3 ? 6 : (KC <= 4 ? 5 : (KC <= 8 ? 3 : 2))) : (KC <= 8 ? 4 : 2))))
 k_msa_wave(MsaParams p){
     extern __shared__ uint8_t smem[];
     __shared__ float sQw[256];

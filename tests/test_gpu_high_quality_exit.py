@@ -1,5 +1,6 @@
-"""GPU tests of the high-quality test in front of the MSA: anchors certain to be corrected as
-high quality without an edit end before their MSA is built.
+"""GPU tests of what spares the MSA stage whole builds: the high-quality test in front of the MSA
+(anchors certain to be corrected as high quality end before their MSA is built) and the
+refinement rounds (removed candidates are taken out of the columns).
 
 Bar: the records equal those of the same pass with intermediates kept, which builds every
 anchor's whole MSA (and is checked against the oracle in tests/test_gpu_parity.py), over the
@@ -85,3 +86,24 @@ def test_learned_records_equal_whole_msa():
     rs = storage(MIXED, "as simulated", 42)
     params, _ = learned.load_classifier()
     assert records(rs, params, correction_type=1) == records(rs, params, correction_type=1, keep_intermediates=1)
+
+
+REFINED = dict(genome_length=20_000, repeat_fraction=0.5, repeat_unit_length=1000, repeat_copies=5)
+
+
+@pytest.mark.parametrize("rule", ["as simulated", None, "lowest"])
+@pytest.mark.parametrize("lengths", [(101, 101), (150, 150), (100, 250), (260, 330), (400, 500)])
+@pytest.mark.parametrize("divergence", [0.004, 0.03])
+def test_refined_records_equal_whole_msa(lengths, rule, divergence):
+    # copies close enough to be each other's candidates: rounds that remove one base's reads
+    rs = storage(dict(REFINED, read_length_min=lengths[0], read_length_max=lengths[1], repeat_divergence=divergence,
+                      coverage=40.0), rule, 43)
+    print(f"[refined {lengths} {rule} {divergence}] reads={rs.n}", flush=True)
+    assert records(rs, estimated_coverage=40.0) == records(rs, estimated_coverage=40.0, keep_intermediates=1)
+
+
+def test_refined_learned_records_equal_whole_msa():
+    rs = storage(dict(REFINED, **MIXED, repeat_divergence=0.01, coverage=40.0), "as simulated", 44)
+    params, _ = learned.load_classifier()
+    opts = dict(correction_type=1, estimated_coverage=40.0)
+    assert records(rs, params, **opts) == records(rs, params, keep_intermediates=1, **opts)
