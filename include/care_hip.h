@@ -62,8 +62,12 @@ typedef struct care_opts {
                                        classifier seam of correctAnchorClf (include/corrector.hpp:
                                        1448-1472) with the MLP of care_hip_set_classifier, and the
                                        classic column rule where its confidence is below 0.9 */
-    int align_variant;              /* staged engine: 0 = one lane per candidate where reads have at
-                                       most 352 bases (else 1), 1 = one wavefront per pair */
+    int align_variant;              /* staged engine: 0 = matrix-core filter (shifts ruled out by a
+                                       fp4 matrix product, the rest counted exactly) where
+                                       max_error_rate is at most 0.3 and the longest read has at
+                                       least 12 shifts beyond the minimum overlap, else one lane per
+                                       candidate (reads of at most 352 bases) or variant 1; 1 = one
+                                       wavefront per pair */
     int use_graphs;                 /* 1 = capture device work into HIP graphs, replayed while their
                                        arguments and buffers hold: the fused engine's pass, or each
                                        pipelined staged batch (see sync_batches) */
@@ -73,7 +77,7 @@ typedef struct care_opts {
     int new_columns_to_correct;     /* --candidateCorrectionNewColumns, 15 */
     int msa_tile;                   /* staged engine: candidates staged into LDS per step of the
                                        one-wavefront MSA, a multiple of 4 in 4..64; 0 = automatic
-                                       (20 with quality scores, else 64) */
+                                       (16 with quality scores, else 64) */
     int seeded_alignment;           /* staged engine, reads of at most 352 bases; not in the reference:
                                        1 = each candidate is aligned only at the strand and shift that
                                        line up the k-mer of the first minhash map it shares with the
@@ -83,8 +87,8 @@ typedef struct care_opts {
                                        hold. Records then differ from the reference's where the scan
                                        would choose another shift or strand; used by the fast learned
                                        form, whose bar is the error rate */
-    int sync_batches;               /* staged engine: 0 = pipelined batches where the lane-per-candidate
-                                       or seeded alignment runs and no candidate correction, dump or
+    int sync_batches;               /* staged engine: 0 = pipelined batches where the matrix, the
+                                       lane-per-candidate or the seeded alignment runs and no candidate correction, dump or
                                        feature output is asked for (no host synchronization inside a
                                        batch: candidate arrays sized from the candidates per anchor
                                        seen, a batch with more is redone; the next batch runs while a

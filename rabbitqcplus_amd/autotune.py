@@ -1,8 +1,8 @@
 """Autotuner: picks the correction schedule for a read set on this GPU by timing.
 
 Candidates are the engine and schedule options the library offers:
-- staged kernels with one lane per candidate in the alignment, or one wavefront per pair;
-- for the lane-per-candidate staged kernels: pipelined batches (no host synchronization
+- staged kernels with the matrix-core alignment, or one wavefront per pair;
+- for the former: pipelined batches (no host synchronization
   inside a batch), the same with each batch captured in a HIP graph, or a host
   synchronization per batch;
 - for the staged kernels, the MSA's candidate tile (candidates staged into LDS per step):

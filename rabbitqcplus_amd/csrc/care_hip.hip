@@ -1,26 +1,29 @@
 // CARE per-anchor error correction on MI355X (gfx950): kernels and C-ABI.
 //
 // Pipeline per batch of anchors (each stage one kernel, all on the context stream):
-//   k_candidates   workgroup per anchor: 48 table lookups, gather of the bucket
-//                  values into LDS, bitonic sort, unique / remove-self / ambiguity
-//                  filter                         (reference include/corrector.hpp:571-650)
-//   k_compact      per-anchor candidate lists -> one dense list + anchor index
+//   k_candidates_wave  wavefront per anchor: the anchor's resolved buckets gathered, distinct
+//                  ids in an LDS hash set, rank sort (reference include/corrector.hpp:571-650);
+//                  k_candidates_over redoes the few anchors with more ids than it takes
+//   k_compact      per-anchor candidate lists -> one dense list
 //   k_pair_flags   mate-pair flags for paired input (include/util.hpp:1016-1200)
-//   k_align        one wavefront per (anchor, candidate): both orientations, lanes over
-//                  shifts on HiLo bit planes held in LDS, popcount mismatches, wave
-//                  argmin with scan-order tie-break (src/cpu_alignment.cpp:32-497,
-//                  include/alignmentorientation.hpp:14-92)
-//   k_msa          workgroup per anchor: orientation + mismatch-ratio filters, MSA
-//                  columns in LDS (thread per column, candidates accumulated in list
-//                  order so float sums match the reference), consensus, up to 5
-//                  refinement rounds, HQ decision, corrected anchor, record encoding
-//                  (include/corrector.hpp:982-1446,1639-1761; src/msa.cpp:9-453,532-734)
+//   k_align_matrix wavefront per anchor: both orientations of 16 candidates at a time, shifts
+//                  ruled out by a matrix product of the lo planes, the others counted exactly
+//                  (align_matrix.hpp; src/cpu_alignment.cpp:32-497,
+//                  include/alignmentorientation.hpp:14-92); scans of every shift
+//                  (k_align_lanes, k_align) where it does not pay
+//   k_msa_wave     wavefront per anchor: filters, the test that ends most anchors before their
+//                  MSA is built (certainHighQuality), MSA columns in registers with candidates
+//                  accumulated in list order so float sums match the reference, up to 5
+//                  refinement rounds, HQ decision, corrected anchor, record
+//                  (include/corrector.hpp:982-1446,1639-1761; src/msa.cpp:9-453,532-734);
+//                  k_msa (workgroup per anchor) for MSAs wider than its registers
 //   k_gather       variable-size records -> contiguous buffer in read-id order
 //
 // Set-up kernels: k_signatures (minhash of every read, include/cpusequencehasher.hpp:
 // 88-125), k_hilo (HiLo planes of every read and its reverse complement,
 // include/sequencehelpers.hpp:646-689), table build = radix sort + run-length
-// encode + bucket filter + open-addressing insert (include/groupbykey.hpp:99-250).
+// encode + bucket filter + open-addressing insert, groups of maps at once
+// (include/groupbykey.hpp:99-250).
 //
 // Float arithmetic follows the reference expression by expression and is compiled
 // without contraction (-ffp-contract=off), so weights, supports and decisions are
@@ -6810,7 +6813,7 @@ static int care_hip_correct_body(care_ctx* ctx, uint64_t first, uint64_t n, size
         ctx->callFirst = first;
     }
     // pipelined batches (no host synchronization inside a batch) for the plain and learned
-    // correction with the lane-per-candidate or seeded alignment; candidate correction,
+    // correction with any alignment but the wavefront per pair; candidate correction,
     // intermediate dumps and feature output synchronize per batch
     const bool pipelined = !fused && !cands && !ctx->o.keep_intermediates && !ctx->featActive && !ctx->o.sync_batches &&
                            (ctx->o.seeded_alignment || matrixAlign(ctx) ||
