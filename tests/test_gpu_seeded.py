@@ -31,6 +31,20 @@ def test_seeded_records_bit_exact(name):
     assert n_g == n_c and d_g == d_c
 
 
+@pytest.mark.parametrize("maps", [1, 2, 3, 4, 5, 6, 7, 47])
+def test_seeded_records_with_any_number_of_maps(maps):
+    """The search takes four maps per step: counts around one step and an odd last step."""
+    s, rs, o = helpers.case("se_higherr_q")
+    o = dict(o, num_hash_maps=maps)
+    print(f"[maps {maps}] reads={rs.n}", flush=True)
+    n_g, d_g = engine.correct_gpu(rs, seeded_alignment=1, **o)
+    cpu = oracle.CareCpu(rs, threads=8, **o)
+    cpu.set_seeded_alignment(True)
+    n_c, d_c = cpu.correct(threads=8)
+    cpu.close()
+    assert n_g == n_c and d_g == d_c
+
+
 @pytest.mark.parametrize("name", ["se_higherr_q", "se_repeats", "pe", "varlen_q"])
 def test_seeded_learned_records_bit_exact(name):
     s, rs, o = helpers.case(name)
