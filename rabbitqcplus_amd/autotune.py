@@ -13,7 +13,7 @@ Candidates are the engine and schedule options the library offers:
 Each candidate corrects the same sample of anchors (after one warm-up pass); the fastest
 (median of `reps` passes) wins. All candidates give byte-identical records, so the choice
 affects speed only. Choices are cached in a JSON file keyed by the device, its compute
-units and the read set's shape (length class, qualities, paired, maps, k).
+units, the read set's length class and the options that select kernels or the schedule.
 """
 from __future__ import annotations
 
@@ -32,15 +32,24 @@ CANDIDATES = [
     {"engine": 2, "waves_per_cu": 8, "use_graphs": 1},
     {"engine": 2, "waves_per_cu": 12, "use_graphs": 1},
 ]
-# MSA tiles swept for the staged kernels (multiples of 4; the default is 20 with quality
-# scores, 64 without)
-TILES_Q = (8, 12, 16, 24, 32)
+# MSA tiles swept for the staged kernels beside the default (multiples of 4; the default is
+# 16 with quality scores, 64 without)
+TILES_Q = (8, 12, 20, 24, 32)
 TILES_NOQ = (16, 32, 48)
 
 
 def candidates(opts) -> list[dict]:
     tiles = TILES_Q if opts.get("use_quality_scores") else TILES_NOQ
     return CANDIDATES + [{"engine": 1, "align_variant": 0, "msa_tile": t} for t in tiles]
+
+# What a cached choice stands for: raised whenever a candidate's options come to mean another
+# kernel or default, so that choices timed before are timed again. 4: align_variant 0 is the
+# matrix-core alignment, pipelined for reads of any length, and the automatic tile is 16.
+CACHE_VERSION = 4
+# Options of the caller that select kernels, or that candidates leave as they are given.
+KEY_OPTIONS = ("use_quality_scores", "paired", "num_hash_maps", "kmerlength", "correction_type", "correct_candidates",
+               "seeded_alignment", "max_error_rate", "min_overlap", "min_overlap_ratio", "batch_size", "use_graphs",
+               "sync_batches", "pipeline_capacity", "msa_tile", "keep_intermediates")
 
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "rabbitqcplus_amd", "autotune.json")
 
@@ -49,8 +58,9 @@ def shape_key(storage, device: int = 0, **opts) -> str:
     name, cus = engine.device_info(device)
     maxlen = int(storage.max_length)
     length_class = 32 * ((maxlen + 31) // 32)
-    return (f"{name}|cu{cus}|len{length_class}|q{int(opts.get('use_quality_scores', 0))}|v3|"
-            f"pe{int(opts.get('paired', 0))}|maps{int(opts.get('num_hash_maps', 48))}|k{int(opts.get('kmerlength', 0))}")
+    o = engine.default_opts(**opts)
+    return "|".join([name, f"cu{cus}", f"len{length_class}", f"v{CACHE_VERSION}"] +
+                    [f"{k}={getattr(o, k):g}" for k in KEY_OPTIONS])
 
 
 def _fits(cand, storage) -> bool:
