@@ -20,10 +20,13 @@
 //
 // Results are those of the scan for every input: the filter passes every admissible shift,
 // whatever order they are counted in. Reads of low complexity pass many shifts; an anchor
-// whose queue takes more than kMatrixBudget per candidate is listed and redone by a scan
+// whose queue takes more than kMatrixBudget per candidate so far (of 16 at least, which ends
+// most of them in their first block, before anything is counted) is listed and redone by a scan
 // (lane per candidate, or for reads of more than 352 bases wavefront per pair), which costs
 // about the same for any sequence: an exact count costs some 4 instructions per shift, the
-// scan of every shift some 150 per candidate.
+// scan of every shift some 150 per candidate. Alignment of reads that are 90% tandem repeats
+// of one or two bases, against the scan alone: 1.13 against 1.28 ms (80,000 of 150 bases), 2.1
+// against 2.35 (68,571 of 100..250), 7.8 against 7.7 (18,461 of 600..700).
 //
 // Measured (MI355X): 1.0M x 150 bases 12.15 -> 4.6 ms against the lane scan, 1.03M reads of
 // 100..250 bases 28.8 -> 8.5 ms, 60,000 of 360..450 bases 7.4 -> 1.2 ms against the wavefront
@@ -145,9 +148,11 @@ k_align_matrix(AlignParams p){
     const int orient = (lane >> 4) & 1;
     const float c1 = 1.0f - 2.0f * p.maxErrorRate;
     int counted = 0;                    // queued shifts so far
-    const int budget = 64 + n * kMatrixBudget;
     auto giveUp = [&](){
-        if(lane == 0) p.list[atomicAdd(p.listCount, 1u)] = uint32_t(ai);
+        if(lane == 0){
+            const ListedAnchors l(p, ai);
+            l.ids[atomicAdd(l.count, 1u)] = uint32_t(ai);
+        }
     };
 
     for(int c0 = 0; c0 < n; c0 += kWave){
@@ -224,6 +229,8 @@ k_align_matrix(AlignParams p){
             const int sigma0 = -((sAlign + max(lcMax - mo, 0) + 31) >> 5);     // blocks sigma0..-1
             const float fLa = c1 * float(La), fLc = c1 * float(lc), fm = -c1 * float(min(La, lc)) - 1.5f;
             int qn = 0;
+            // queued shifts that the candidates up to this block's last may have
+            const int budget = max(min(c0 + (b + 1) * kMatrixCands, n), kMatrixCands) * kMatrixBudget;
 
             // counts the queued shifts exactly, two lanes per shift
             auto flush = [&](){

@@ -792,8 +792,8 @@ struct AlignParams {
     // seeded alignment: every read's bucket (offset, count) and seed per map, read-major
     const uint2* bucketOf; const uint16_t* seeds; int M; int k; int thr;
     // anchors (indices within the batch) that the matrix kernel leaves to a scan of every
-    // shift, and their number
-    uint32_t* list; uint32_t* listCount;
+    // shift (ListedAnchors); null where it does not run
+    uint32_t* listed;
 };
 
 struct ShdResult { int score, overlap, shift, nOps, valid; };
@@ -1040,22 +1040,52 @@ k_align(AlignParams p){
     }
 }
 
-// The pairs of the listed anchors: workgroups stride over the list, one anchor at a time.
-__global__ void __launch_bounds__(kBlock)
-k_align_listed(AlignParams p){
-    __shared__ uint2 planes[kAlignWaves][6][kMaxHiLoWords + 1];
-    const int wave = threadIdx.x / kWave;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int count = int(*p.listCount);
-    for(int b = blockIdx.x; b < count; b += gridDim.x){
-        const int i = int(p.list[b]);
-        const uint32_t beg = p.offsets[i], end = p.offsets[i + 1];
-        for(uint64_t base = beg; base < end; base += kAlignWaves){
-            const uint64_t c = base + uint64_t(wave);
-            const bool active = c < end;
-            alignPair(p, planes[wave], active, p.b0 + uint64_t(i), active ? p.ids[c] : 0u, c, lane);
-        }
+// The listed anchors of a batch: lists by the low bits of the anchor's index, each with its
+// count and the number of work items taken from it in a 64-byte line of its own (0 before the
+// batch's alignment), then the anchors' indices. One counter for all served 66,000 anchors of
+// a batch one after another: k_align_matrix 435 us, 290 us with 64.
+constexpr int kAnchorLists = 64;
+constexpr int kListLine = 16;                           // words
+constexpr int kListHeader = kAnchorLists * kListLine;   // words
+struct ListedAnchors {
+    uint32_t* count; uint32_t* taken; uint32_t* ids;
+    __device__ __forceinline__ ListedAnchors(const AlignParams& p, int i){
+        const int s = i & (kAnchorLists - 1);
+        count = p.listed + s * kListLine;
+        taken = count + 1;
+        ids = p.listed + kListHeader + s * ((p.B + kAnchorLists - 1) / kAnchorLists);
     }
+};
+
+// f(anchor, part) for the listed anchors and parts 0..PARTS-1, each by one wavefront of a grid
+// of single wavefronts, which take them as they get free: anchors differ in candidates, and
+// with fixed strides the others waited for the last (k_align_listed 9.5 -> 7.3 ms on 18,461
+// reads of 600..700 bases, k_align_lanes<5> 1.02 -> 0.85 ms on 80,000 of 150).
+template<int PARTS, class F>
+__device__ __forceinline__ void forListed(const AlignParams& p, F&& f){
+    const ListedAnchors l(p, int(blockIdx.x) % min(p.B, kAnchorLists));
+    const uint32_t items = *l.count * uint32_t(PARTS);
+    if(items == 0) return;
+    for(;;){
+        uint32_t u = 0;
+        if(threadIdx.x == 0) u = atomicAdd(l.taken, 1u);
+        u = uint32_t(__builtin_amdgcn_readfirstlane(int(u)));
+        if(u >= items) return;
+        f(int(l.ids[u / PARTS]), int(u % PARTS));
+    }
+}
+
+// The pairs of the listed anchors, every kListParts-th of an anchor's by one wavefront (about six
+// of the pairs of a read set of 30x at a time).
+constexpr int kListParts = 16;
+__global__ void __launch_bounds__(kWave)
+k_align_listed(AlignParams p){
+    __shared__ uint2 planes[6][kMaxHiLoWords + 1];
+    forListed<kListParts>(p, [&](int i, int part){
+        const uint64_t end = p.offsets[i + 1];
+        for(uint64_t c = uint64_t(p.offsets[i]) + uint64_t(part); c < end; c += kListParts)
+            alignPair(p, planes, true, p.b0 + uint64_t(i), p.ids[c], c, threadIdx.x);
+    });
 }
 
 // ---------------------------------------------------------------- alignment, lane per candidate
@@ -1394,13 +1424,12 @@ __device__ __forceinline__ void alignAnchor(const AlignParams& p, int i){
 }
 
 // One wavefront per anchor of the batch (a grid of p.B), its candidates in chunks of 64
-// lanes; LISTED: wavefronts striding over the listed anchors.
+// lanes; LISTED: the listed anchors.
 template<int WM, bool LISTED>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WM <= 5 ? 8 : 1)))
 k_align_lanes(AlignParams p){
     if constexpr(LISTED){
-        const int count = int(*p.listCount);
-        for(int b = blockIdx.x; b < count; b += gridDim.x) alignAnchor<WM>(p, int(p.list[b]));
+        forListed<1>(p, [&](int i, int){ alignAnchor<WM>(p, i); });
     }else{
         if(int(blockIdx.x) < p.B) alignAnchor<WM>(p, batchAnchor(p.order, p.B));
     }
@@ -3613,14 +3642,14 @@ __global__ void k_zero_u32(uint32_t* v, int n){
 // Start of a pipelined batch: candidate counts and record sizes 0, the counts of both redo
 // lists and the status words 0 (one launch; five cost 20 us of a 260 us pass over 6,000 reads).
 __global__ void __launch_bounds__(256) k_batch_init(uint32_t* __restrict__ uniq, uint32_t* __restrict__ recBytes, int B,
-                                                    uint32_t* __restrict__ overCount, uint32_t* __restrict__ listCount,
+                                                    uint32_t* __restrict__ overCount, uint32_t* __restrict__ listed,
                                                     uint32_t* __restrict__ status){
     FOR_GRID(i, B + 1){ uniq[i] = 0u; recBytes[i] = 0u; }
     if(blockIdx.x == 0){
         if(threadIdx.x < kStatusWords) status[threadIdx.x] = 0u;
         if(threadIdx.x == 0) *overCount = 0u;
-        if(threadIdx.x == 1 && listCount) *listCount = 0u;
     }
+    if(listed) FOR_GRID(i, kListHeader){ listed[i] = 0u; }
 }
 
 // Capacity check of a pipelined batch (status words as slotStatus lays them out): the flag and
@@ -4173,7 +4202,7 @@ void fillAlignCommon(const care_ctx* ctx, AlignParams& ap){
     ap.maxLen = ctx->maxLen;
     ap.eExact = errorBoundAsInteger(ap.maxErrorRate, ctx->maxLen, ap.eMul, ap.ePre) ? 1 : 0;
     if(!ap.eExact){ ap.eMul = 0; ap.ePre = 0; }
-    ap.list = nullptr; ap.listCount = nullptr;
+    ap.listed = nullptr;
     ap.order = nullptr;
     ap.bucketOf = ctx->bucketOf.as<uint2>(); ap.seeds = ctx->seeds.as<uint16_t>();
     ap.M = ctx->M; ap.k = ctx->k; ap.thr = ctx->thr;
@@ -4479,10 +4508,9 @@ bool matrixAlign(const care_ctx* ctx){
 // The list of anchors the matrix kernel leaves to a scan, for batches of at most B.
 hipError_t prepareAlignList(care_ctx* ctx, int B, AlignParams& ap){
     if(!matrixAlign(ctx)) return hipSuccess;
-    const hipError_t e = ctx->alignOver.ensure(size_t(B) * 4 + 16);
+    const hipError_t e = ctx->alignOver.ensure((size_t(kListHeader) + size_t(B) + kAnchorLists) * 4);
     if(e != hipSuccess) return e;
-    ap.listCount = ctx->alignOver.as<uint32_t>();
-    ap.list = ctx->alignOver.as<uint32_t>() + 4;
+    ap.listed = ctx->alignOver.as<uint32_t>();
     return hipSuccess;
 }
 
@@ -4499,7 +4527,7 @@ hipError_t launchAlignLanes(const AlignParams& ap, int grid, int wm, hipStream_t
 }
 
 // The alignment kernel of a staged batch: the seeded kernel (seeded alignment), the matrix
-// kernel followed by the scan of the anchors it listed (*ap.listCount is 0 before), the
+// kernel followed by the scan of the anchors it listed (its lists are empty before), the
 // lane-per-candidate kernel (wm > 0), or the wavefront-per-pair kernel over `total` pairs.
 hipError_t launchAlign(const care_ctx* ctx, const AlignParams& ap, int B, uint32_t total, int wm, hipStream_t st){
     if(ctx->o.seeded_alignment){
@@ -4528,7 +4556,7 @@ hipError_t launchAlign(const care_ctx* ctx, const AlignParams& ap, int B, uint32
         const hipError_t e = hipGetLastError();
         if(e != hipSuccess) return e;
         if(alignLaneWords(ctx->W) > 0) return launchAlignLanes<true>(ap, std::min(B, 8192), alignLaneWords(ctx->W), st);
-        k_align_listed<<<std::min(B, 8192), kBlock, 0, st>>>(ap);
+        k_align_listed<<<int(std::min<int64_t>(int64_t(B) * kListParts, 8192)), kWave, 0, st>>>(ap);
         return hipGetLastError();
     }
     if(wm > 0) return launchAlignLanes<false>(ap, B, wm, st);
@@ -4673,7 +4701,7 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     ap.offsets = ctx->offsets.as<uint32_t>(); ap.B = B; ap.maxLen = ctx->maxLen;
     ap.order = order;
     HIPCHECK(prepareAlignList(ctx, B, ap));
-    if(ap.listCount) k_zero_u32<<<1, 64, 0, st>>>(ap.listCount, 1);
+    if(ap.listed) k_zero_u32<<<kListHeader / 256, 256, 0, st>>>(ap.listed, kListHeader);
     if(total) HIPCHECK(launchAlign(ctx, ap, B, total, wm, st));
     HIPCHECK(hipEventRecord(ctx->ev[2], st));
 
@@ -4814,7 +4842,7 @@ hipError_t enqueueStaged(care_ctx* ctx, const StagedLaunch& L, bool events){
 #define ENQE(expr) do { e = (expr); if(e != hipSuccess) return e; } while(0)
     uint32_t* overCount = reinterpret_cast<uint32_t*>(ctx->candOver.as<uint8_t>() + size_t(B) * 4);
     ENQ((k_batch_init<<<gridFor(uint64_t(B) + 1, 256), 256, 0, st>>>(L.cp.uniq, ctx->recBytes.as<uint32_t>(), B, overCount,
-                                                                     L.ap.listCount, status)));
+                                                                     L.ap.listed, status)));
     ENQ((k_candidates_wave<<<B, kWave, L.waveLds, st>>>(L.cp, ctx->candOver.as<uint32_t>(), overCount)));
     ENQ((k_candidates_over<<<std::min(B, 4096), kBlock, L.candLds, st>>>(L.cp, ctx->candOver.as<uint32_t>(), overCount)));
     ENQ((k_add_gathered<<<dim3(uint32_t((B + kAddPerBlock - 1) / kAddPerBlock), 2), kBlock, 0, st>>>(
