@@ -3679,23 +3679,23 @@ __global__ void k_cap_check(uint64_t cap, uint32_t* __restrict__ offsets, int B,
 // waves), finds those with a record by ballot and copies them one after another, lanes over
 // bytes; wavefronts stride over the batch. Most anchors have no record: a workgroup per anchor
 // spent 212 us on 1.0M anchors with 130,000 records, where this takes about 20, and a wave per
-// candidate entry 700 us on 10.0M entries with 707,000 records, about 170. `count` (may be
-// null) receives the number of records.
+// candidate entry 700 us on 10.0M entries with 707,000 records, about 170. Returns the wave's
+// records.
 constexpr int kGatherGrid = 4096;
 constexpr uint64_t kGatherSmall = uint64_t(kGatherGrid) * (kBlock / kWave) * kWave / 8;
 template<class Size, class Src>
-__device__ __forceinline__ void copyRecords(uint64_t n, const Size* __restrict__ size, const uint64_t* __restrict__ off,
-                                              uint8_t* __restrict__ out, unsigned long long* count, Src&& src){
+__device__ __forceinline__ uint32_t copyRecords(uint64_t n, const Size* __restrict__ size, const uint64_t* __restrict__ off,
+                                                uint8_t* __restrict__ out, Src&& src){
     const int lane = threadIdx.x & (kWave - 1);
     const uint64_t waves = uint64_t(gridDim.x) * (blockDim.x / kWave);
     const uint64_t per = n <= kGatherSmall ? 8 : kWave;
-    unsigned long long found = 0;
+    uint32_t found = 0;
     for(uint64_t base = (uint64_t(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave) * per; base < n;
         base += waves * per){
         const uint64_t e = base + uint64_t(lane);
         const uint32_t nb = uint64_t(lane) < per && e < n ? uint32_t(size[e]) : 0u;
         uint64_t mask = __ballot(nb != 0);
-        found += (unsigned long long)(__popcll(mask));
+        found += uint32_t(__popcll(mask));
         const uint64_t at = nb ? off[e] : 0;
         const uint64_t from = nb ? src(e) : 0;
         while(mask){
@@ -3710,29 +3710,24 @@ __device__ __forceinline__ void copyRecords(uint64_t n, const Size* __restrict__
             for(uint32_t q = lane; q < bytes; q += kWave) out[o + q] = s[q];
         }
     }
-    if(count && lane == 0 && found) atomicAdd(count, found);
+    return found;
 }
 
 __global__ void __launch_bounds__(kBlock)
 k_gather(const uint8_t* slots, int slotBytes, const uint32_t* recBytes, const uint64_t* outOff, uint8_t* out, int B,
-         unsigned long long* count, uint32_t* status, const int* error){
+         uint32_t* status, const int* error){
     // a pipelined batch's record bytes and error flag, beside its other status words
     if(status && blockIdx.x == 0 && threadIdx.x == 0){
         *reinterpret_cast<uint64_t*>(status + 8) = outOff[B];
         status[10] = uint32_t(*error);
     }
-    copyRecords(uint64_t(B), recBytes, outOff, out, count,
-                  [&](uint64_t i){ return reinterpret_cast<uint64_t>(slots + i * uint64_t(slotBytes)); });
+    copyRecords(uint64_t(B), recBytes, outOff, out,
+                [&](uint64_t i){ return reinterpret_cast<uint64_t>(slots + i * uint64_t(slotBytes)); });
 }
 
-__global__ void k_widen(const uint32_t* in, uint64_t* out, int n){
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i < n) out[i] = in[i];
-}
-
-// k_widen over kWidenPerBlock sizes per 256-thread workgroup, and the number of nonzero
-// sizes (records) added to *count: wave ballots summed in LDS, one global atomic per
-// workgroup.
+// Record sizes widened to 64 bits, kWidenPerBlock per 256-thread workgroup, and the number of
+// nonzero sizes (records) added to *count: wave ballots summed in LDS, one global atomic per
+// workgroup (atomics on one address take some 12 ns each, one after another).
 constexpr int kWidenPerBlock = 1024;
 __global__ void __launch_bounds__(256) k_widen_count(const uint32_t* __restrict__ in, uint64_t* __restrict__ out, int n,
                                                      unsigned long long* __restrict__ count){
@@ -3796,11 +3791,17 @@ __global__ void k_insertion_order(const uint32_t* __restrict__ recBytes, const u
     }
 }
 
-// One wavefront per entry: copies its record to its offset in the batch's stream.
+// Copies the entries' records to their offsets in the batch's stream and adds their number to *count.
 __global__ void __launch_bounds__(256) k_gather_entries(const uint64_t* __restrict__ size, const uint64_t* __restrict__ src,
                                                         const uint64_t* __restrict__ off, uint8_t* __restrict__ out,
                                                         uint64_t entries, unsigned long long* count){
-    copyRecords(entries, size, off, out, count, [&](uint64_t e){ return src[e]; });
+    __shared__ unsigned blockCount;
+    if(threadIdx.x == 0) blockCount = 0;
+    __syncthreads();
+    const uint32_t found = copyRecords(entries, size, off, out, [&](uint64_t e){ return src[e]; });
+    if((threadIdx.x & (kWave - 1)) == 0 && found) atomicAdd(&blockCount, found);
+    __syncthreads();
+    if(threadIdx.x == 0 && blockCount) atomicAdd(count, (unsigned long long)blockCount);
 }
 
 // ---------------------------------------------------------------- host side
@@ -4227,19 +4228,23 @@ dim3 gatherGrid(uint64_t n){
     return dim3(uint32_t(std::min<uint64_t>((n + per - 1) / per, kGatherGrid)));
 }
 unsigned long long* recordCounter(care_ctx* ctx){ return ctx->counters.as<unsigned long long>() + 6; }
+// Its copy in the context's pinned words.
+uint64_t* recordCount(care_ctx* ctx){ return reinterpret_cast<uint64_t*>(reinterpret_cast<uint8_t*>(ctx->pinned) + 16); }
 
 // Record compaction, device part: record sizes widened and scanned into byte offsets,
-// then the total and the error flag copied into the context's pinned host words (no host
-// synchronization; capturable). Uses the preallocated scan workspace only.
+// then the total, the error flag and the number of records (whose counter is 0 before) copied
+// into the context's pinned host words (no host synchronization; capturable). Uses the preallocated scan workspace only.
 int recordsDevicePart(care_ctx* ctx, int B){
     hipStream_t st = ctx->stream;
-    k_widen<<<(B + 1 + 255) / 256, 256, 0, st>>>(ctx->recBytes.as<uint32_t>(), ctx->recOff64.as<uint64_t>(), B + 1);
+    k_widen_count<<<(B + 1 + kWidenPerBlock - 1) / kWidenPerBlock, 256, 0, st>>>(
+        ctx->recBytes.as<uint32_t>(), ctx->recOff64.as<uint64_t>(), B + 1, recordCounter(ctx));
     HIPCHECK(hipGetLastError());
     size_t tb = ctx->scanTmp.bytes;
     HIPCHECK(hipcub::DeviceScan::ExclusiveSum(ctx->scanTmp.p, tb, ctx->recOff64.as<uint64_t>(), ctx->recOff.as<uint64_t>(), B + 1, st));
     HIPCHECK(hipMemcpyAsync(ctx->pinned, ctx->recOff.as<uint64_t>() + B, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipMemcpyAsync(reinterpret_cast<uint8_t*>(ctx->pinned) + 8, ctx->counters.as<int>() + 2, 4,
                             hipMemcpyDeviceToHost, st));
+    HIPCHECK(hipMemcpyAsync(recordCount(ctx), recordCounter(ctx), 8, hipMemcpyDeviceToHost, st));
     return CARE_OK;
 }
 
@@ -4262,18 +4267,14 @@ int recordsFinish(care_ctx* ctx, int B, int slotBytes, HostRecords& out, size_t&
     std::memcpy(&errFlag, reinterpret_cast<uint8_t*>(ctx->pinned) + 8, 4);
     if(errFlag) return ctx->fail(CARE_EINVAL, "MSA column bound exceeded");
     HIPCHECK(ctx->outBuf.ensure(std::max<uint64_t>(outBytes, 1)));
-    unsigned long long* recs = recordCounter(ctx);
-    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(recs), 2);
     k_gather<<<gatherGrid(B), kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), slotBytes, ctx->recBytes.as<uint32_t>(),
-                                               ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B, recs, nullptr, nullptr);
+                                               ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B, nullptr, nullptr);
     HIPCHECK(hipGetLastError());
     const size_t old = out.size();
     HIPCHECK(out.resize(old + outBytes));
     if(outBytes) HIPCHECK(hipMemcpyAsync(out.data() + old, ctx->outBuf.p, outBytes, hipMemcpyDeviceToHost, st));
-    unsigned long long records = 0;
-    HIPCHECK(hipMemcpyAsync(&records, recs, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));
-    outRecords += size_t(records);
+    outRecords += size_t(*recordCount(ctx));
     return CARE_OK;
 }
 
@@ -4311,9 +4312,9 @@ int runFused(care_ctx* ctx, uint64_t first, uint64_t n, HostRecords& out, size_t
     fp.m.slots = ctx->slots.as<uint8_t>(); fp.m.slotBytes = slotBytes; fp.m.recBytes = ctx->recBytes.as<uint32_t>();
     fp.m.error = ctx->counters.as<int>() + 2;
     fp.c.b0 = first; fp.c.B = B; fp.c.raw = nullptr; fp.c.uniq = nullptr; fp.c.gathered = ctx->counters.as<unsigned long long>();
-    // counters: [0,8) gathered bucket values, [8,12) error flag, [16,20) work counter,
-    // [24,32) candidates aligned, [32,40) decision columns written out
-    fp.counter = ctx->counters.as<uint32_t>() + 4;
+    // counters: [0,8) gathered bucket values, [8,12) error flag, [24,32) candidates aligned,
+    // [32,40) decision columns written out, [48,56) records, [56,60) work counter
+    fp.counter = ctx->counters.as<uint32_t>() + 14;
     fp.aligned = ctx->counters.as<unsigned long long>() + 3;
     fp.first = first;
     fp.units = uint32_t(units);
@@ -4342,7 +4343,7 @@ int runFused(care_ctx* ctx, uint64_t first, uint64_t n, HostRecords& out, size_t
     auto enqueue = [&]() -> hipError_t {
         // recBytes[B] must read as zero for the exclusive scan; the kernel writes [0, B)
         k_zero_u32<<<1, 64, 0, st>>>(ctx->recBytes.as<uint32_t>() + B, 1);
-        k_zero_u32<<<1, 64, 0, st>>>(ctx->counters.as<uint32_t>() + 4, 1);
+        k_zero_u32<<<1, 64, 0, st>>>(ctx->counters.as<uint32_t>() + 12, 3);
         void* args[] = {&fp};
         hipError_t e = hipLaunchKernel(kernelFor(), dim3(uint32_t(G)), dim3(kWave), args, lds, st);
         if(e != hipSuccess) return e;
@@ -4443,7 +4444,6 @@ int gatherInsertionOrder(care_ctx* ctx, uint64_t b0, int B, uint32_t total, int 
     if(errFlag) return ctx->fail(CARE_EINVAL, "MSA column bound exceeded in batch at %llu", (unsigned long long)b0);
     HIPCHECK(ctx->outBuf.ensure(std::max<uint64_t>(outBytes, 1)));
     unsigned long long* recs = recordCounter(ctx);
-    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(recs), 2);
     k_gather_entries<<<gatherGrid(entries), 256, 0, st>>>(
         ctx->insSize.as<uint64_t>(), ctx->insSrc.as<uint64_t>(), ctx->insOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(),
         entries, recs);
@@ -4451,8 +4451,7 @@ int gatherInsertionOrder(care_ctx* ctx, uint64_t b0, int B, uint32_t total, int 
     const size_t old = out.size();
     HIPCHECK(out.resize(old + outBytes));
     if(outBytes) HIPCHECK(hipMemcpyAsync(out.data() + old, ctx->outBuf.p, outBytes, hipMemcpyDeviceToHost, st));
-    unsigned long long records = 0;
-    HIPCHECK(hipMemcpyAsync(&records, recs, 8, hipMemcpyDeviceToHost, st));
+    HIPCHECK(hipMemcpyAsync(recordCount(ctx), recs, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipEventRecord(ctx->ev[4], st));
     HIPCHECK(hipStreamSynchronize(st));
     float ms = 0;
@@ -4462,7 +4461,7 @@ int gatherInsertionOrder(care_ctx* ctx, uint64_t b0, int B, uint32_t total, int 
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[2], ctx->ev[3])); ctx->t.msa_ms += ms; ctx->t.msa_kernel_ms += ms;
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[3], ctx->ev[4])); ctx->t.output_ms += ms;
     ctx->t.candidates += total;
-    outRecords += size_t(records);
+    outRecords += size_t(*recordCount(ctx));
     return CARE_OK;
 }
 
@@ -4649,7 +4648,7 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     HIPCHECK(hipGetLastError());
     // the batch's candidate pairs in 64 bits: list offsets and indices are 32-bit
     unsigned long long* pairs64 = ctx->counters.as<unsigned long long>() + 5;
-    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(pairs64), 2);
+    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(pairs64), 4);      // and the record counter behind it
     k_add_gathered<<<(B + kAddPerBlock - 1) / kAddPerBlock, kBlock, 0, st>>>(ctx->uniq.as<uint32_t>(), B, pairs64, nullptr, nullptr);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(ctx->ev[5], st));
@@ -4774,7 +4773,8 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     }
 
     // record compaction
-    k_widen<<<(B + 1 + 255) / 256, 256, 0, st>>>(ctx->recBytes.as<uint32_t>(), ctx->recOff64.as<uint64_t>(), B + 1);
+    k_widen_count<<<(B + 1 + kWidenPerBlock - 1) / kWidenPerBlock, 256, 0, st>>>(
+        ctx->recBytes.as<uint32_t>(), ctx->recOff64.as<uint64_t>(), B + 1, recordCounter(ctx));
     HIPCHECK(hipGetLastError());
     HIPCHECK(ctx->recOff.ensure(size_t(B + 1) * 8));
     tb = 0;
@@ -4786,23 +4786,20 @@ int runBatch(care_ctx* ctx, uint64_t b0, int B, HostRecords& out, size_t& outRec
     int errFlag = 0;
     HIPCHECK(hipMemcpyAsync(&outBytes, ctx->recOff.as<uint64_t>() + B, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipMemcpyAsync(&errFlag, ctx->counters.as<int>() + 2, 4, hipMemcpyDeviceToHost, st));
+    HIPCHECK(hipMemcpyAsync(recordCount(ctx), recordCounter(ctx), 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipStreamSynchronize(st));
     if(errFlag) return ctx->fail(CARE_EINVAL, "MSA column bound exceeded in batch at %llu", (unsigned long long)b0);
     HIPCHECK(ctx->outBuf.ensure(std::max<uint64_t>(outBytes, 1)));
-    unsigned long long* recs = recordCounter(ctx);
-    k_zero_u32<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(recs), 2);
     k_gather<<<gatherGrid(B), kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), slotBytes, ctx->recBytes.as<uint32_t>(),
-                                               ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B, recs, nullptr, nullptr);
+                                               ctx->recOff.as<uint64_t>(), ctx->outBuf.as<uint8_t>(), B, nullptr, nullptr);
     HIPCHECK(hipGetLastError());
     const size_t old = out.size();
     HIPCHECK(out.resize(old + outBytes));
     if(outBytes) HIPCHECK(hipMemcpyAsync(out.data() + old, ctx->outBuf.p, outBytes, hipMemcpyDeviceToHost, st));
-    unsigned long long records = 0;
-    HIPCHECK(hipMemcpyAsync(&records, recs, 8, hipMemcpyDeviceToHost, st));
     HIPCHECK(hipEventRecord(ctx->ev[4], st));
     HIPCHECK(hipStreamSynchronize(st));
 
-    outRecords += size_t(records);
+    outRecords += size_t(*recordCount(ctx));
     float ms;
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1])); ctx->t.candidates_ms += ms;
     HIPCHECK(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[5])); ctx->t.cand_kernel_ms += ms;
@@ -4882,7 +4879,7 @@ hipError_t enqueueStaged(care_ctx* ctx, const StagedLaunch& L, bool events){
     tb = ctx->scanTmp.bytes;
     ENQE(hipcub::DeviceScan::ExclusiveSum(ctx->scanTmp.p, tb, ctx->recOff64.as<uint64_t>(), ctx->recOff.as<uint64_t>(), B + 1, st));
     ENQ((k_gather<<<gatherGrid(B), kBlock, 0, st>>>(ctx->slots.as<uint8_t>(), L.slotBytes, ctx->recBytes.as<uint32_t>(),
-                                                    ctx->recOff.as<uint64_t>(), ctx->pipeOut[L.slot].as<uint8_t>(), B, nullptr,
+                                                    ctx->recOff.as<uint64_t>(), ctx->pipeOut[L.slot].as<uint8_t>(), B,
                                                     status, ctx->counters.as<int>() + 2)));
     uint8_t* pw = slotPinned(ctx, L.slot);
     ENQE(hipMemcpyAsync(pw, status, kStatusWords * 4, hipMemcpyDeviceToHost, st));
