@@ -33,6 +33,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "care_hip.h"
+#include "msa_bounds.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -2813,12 +2814,13 @@ template<int KC>
 __device__ __forceinline__ bool decidedWithin(const MsaParams& p, const WaveMsa<KC>& m, float weightError, int La){
     float least = 2.0f, leastHi = 2.0f;
     int sum = 0, off = 0, mincov = INT_MAX;
-    bool differs = false, near = false;
+    bool differs = false, near = false, unknown = false;
     #pragma unroll
     for(int k = 0; k < KC; k++){
         if(!((m.isAnchor >> k) & 1u)) continue;
         const float colW = m.w[k][0] + m.w[k][1] + m.w[k][2] + m.w[k][3];
-        const float e = fminf(6.0f * weightError / fmaxf(colW, 1e-3f) + 1e-6f, 1.0f);
+        const float e = supportError(colW, weightError);
+        if(e > 1.0f){ unknown = true; continue; }
         const float s = m.sup[k];
         least = fminf(least, s - e);
         leastHi = fminf(leastHi, s + e);
@@ -2831,6 +2833,7 @@ __device__ __forceinline__ bool decidedWithin(const MsaParams& p, const WaveMsa<
             near |= countOf(m, k, ob) <= 2 && fabsf(s - 0.90f) <= e;
         }
     }
+    if(__ballot(unknown) != 0) return false;
     // (supports are at most 1 and La at most 1024: the sums fit 31 bits)
     const float scale = 1.0f / (1048576.0f * float(La));
     const float avg = float(waveReduce(sum, OpSum(), 0)) * scale;
@@ -3152,14 +3155,11 @@ __device__ __forceinline__ void msaAnchorWave(const MsaParams& p, const AnchorLi
             bool close = false;
             #pragma unroll
             for(int k = 0; k < KC; k++){
+                int bases = 4;
                 #pragma unroll
-                for(int b = 0; b < 4; b++) if(countOf(m, k, b) == 0) m.w[k][b] = 0.0f;
-                if((m.isAnchor >> k) & 1u){
-                    const float w01 = fmaxf(m.w[k][0], m.w[k][1]), v01 = fminf(m.w[k][0], m.w[k][1]);
-                    const float w23 = fmaxf(m.w[k][2], m.w[k][3]), v23 = fminf(m.w[k][2], m.w[k][3]);
-                    const float first = fmaxf(w01, w23), second = fmaxf(fminf(w01, w23), fmaxf(v01, v23));
-                    close |= second != 0.0f && first - second <= 2.0f * weightError + 1e-6f;
-                }
+                for(int b = 0; b < 4; b++) if(countOf(m, k, b) == 0){ m.w[k][b] = 0.0f; bases--; }
+                if((m.isAnchor >> k) & 1u)
+                    close |= !consensusCertain(m.w[k][0], m.w[k][1], m.w[k][2], m.w[k][3], bases, weightError);
             }
             if(__ballot(close) == 0){
                 finishColumns<KC, AO>(m, lane);
