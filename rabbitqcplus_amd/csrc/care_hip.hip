@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include "bucket_rows.hpp"
 #include "care_hip.h"
 #include "msa_bounds.hpp"
 
@@ -1511,19 +1512,13 @@ k_align_seeded(AlignParams p){
         if(c >= n) break;
         const uint32_t id = p.ids[beg + c];
         const int Lc = p.len[id];
-        // first map whose kept bucket holds both reads (equal offset and count); rows of
-        // M (even) buckets are 16-byte aligned
+        // first map whose kept bucket holds both reads (equal offset and count)
         const uint2* cbk = p.bucketOf + uint64_t(id) * uint64_t(M);
         int m = M;
         for(int q = 0; 2 * q < M && m == M; q += kSeedPairs){
             uint4 x[kSeedPairs];
             #pragma unroll
-            for(int t = 0; t < kSeedPairs; t++){
-                const int u = 2 * (q + t);
-                x[t] = make_uint4(0u, 0u, 0u, 0u);
-                if(u + 1 < M) x[t] = *reinterpret_cast<const uint4*>(cbk + u);
-                else if(u < M){ const uint2 y = cbk[u]; x[t] = make_uint4(y.x, y.y, 0u, 0u); }
-            }
+            for(int t = 0; t < kSeedPairs; t++) x[t] = bucketPair(cbk, 2 * (q + t), M);
             #pragma unroll
             for(int t = kSeedPairs - 1; t >= 0; t--){       // the lowest map of the step is kept
                 const int u = 2 * (q + t);
