@@ -3987,8 +3987,10 @@ int buildTables(care_ctx* ctx){
                                                    (uint32_t*)nullptr, (int*)nullptr, int(items), st));
     HIPCHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb3, (const uint32_t*)nullptr, (uint32_t*)nullptr, int(items), st));
     const size_t tempBytes = std::max({tb1, tb2, tb3, size_t(256)});
-    // one workspace, kept by the context for the next reads (its size is bounded by
-    // kGroupItems or one map, about 50 bytes per item)
+    // one workspace of about 40 bytes per item, kept by the context for the next reads up to
+    // kGroupItems; that of a larger map goes back when the tables are built, or the passes'
+    // batches would be sized from what it leaves
+    struct Bounded { DBuf& b; bool keep; ~Bounded(){ if(!keep) b.release(); } } bounded{ctx->tableTmp, items <= kGroupItems};
     auto up = [](size_t b){ return (b + 255) & ~size_t(255); };
     const size_t b8 = up(items * 8), b4 = up(items * 4);
     HIPCHECK(ctx->tableTmp.ensure((group > 1 ? 3 : 2) * b8 + 3 * b4 + 512 + up(tempBytes)));
