@@ -25,6 +25,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <random>
@@ -606,14 +607,16 @@ static int care_mlp_train_body(care_mlp* h, int epochs, int batch, float lr, uin
     k_fill<<<(std::max(epochs, 1) + 255) / 256, 256, 0, st>>>(h->epochLoss.as<float>(), std::max(epochs, 1), 0.0f);
     const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
     std::mt19937_64 rng(seed);
-    std::vector<uint32_t> perm(n);
-    auto shuffle = [&](){
-        std::iota(perm.begin(), perm.end(), 0u);
-        std::shuffle(perm.begin(), perm.end(), rng);
+    // two arrays in turn: an epoch's order stays as it is until its copy is known to be over
+    std::unique_ptr<uint32_t[]> perm[2];
+    auto shuffle = [&](std::unique_ptr<uint32_t[]>& v){
+        if(!v) v.reset(new uint32_t[n]);
+        std::iota(v.get(), v.get() + n, 0u);
+        std::shuffle(v.get(), v.get() + n, rng);
     };
-    if(epochs > 0) shuffle();
+    if(epochs > 0) shuffle(perm[0]);
     for(int ep = 0; ep < epochs; ep++){
-        MCHECK(hipMemcpyAsync(h->perm.p, perm.data(), n * 4, hipMemcpyHostToDevice, st));
+        MCHECK(hipMemcpyAsync(h->perm.p, perm[ep & 1].get(), n * 4, hipMemcpyHostToDevice, st));
         for(size_t b = 0; b < batches; b++){
             const int rows = int(std::min<size_t>(size_t(bsz), n - b * bsz));
             k_gather_rows<<<(rows * kIn + 255) / 256, 256, 0, st>>>(h->Xall.as<float>(), h->yall.as<float>(),
@@ -633,9 +636,8 @@ static int care_mlp_train_body(care_mlp* h, int epochs, int batch, float lr, uin
                                                      h->v.as<float>(), lr, beta1, beta2, eps, c1, c2);
             MCHECK(hipGetLastError());
         }
-        // the next epoch's order, drawn while this one runs (the copy above left the host
-        // array when it returned: it is pageable memory)
-        if(ep + 1 < epochs) shuffle();
+        // the next epoch's order, drawn while this one runs
+        if(ep + 1 < epochs) shuffle(perm[(ep + 1) & 1]);
         // the permutation buffer is rewritten next epoch: wait for this epoch's gathers
         MCHECK(hipStreamSynchronize(st));
     }
