@@ -30,8 +30,8 @@
 //
 // Measured (MI355X): 1.0M x 150 bases 12.15 -> 4.6 ms against the lane scan, 1.03M reads of
 // 100..250 bases 28.8 -> 8.5 ms, 60,000 of 360..450 bases 7.4 -> 1.2 ms against the wavefront
-// per pair. At 150 bases: 2.9k vector and 1.5k scalar instructions per anchor (1.1 and 0.6
-// per clock and CU at 5.9 waves per SIMD), matrix cores busy a fifth of the time; bound by
+// per pair. At 150 bases: 3.1k vector and 1.6k scalar instructions per anchor (1.1 and 0.6
+// per clock and CU at 5.8 waves per SIMD), matrix cores busy a fifth of the time; bound by
 // instruction issue and by the latency of its LDS and accumulator reads.
 //
 // Position order inside a 64-deep step is free as long as both operands share it: dword i

@@ -3674,7 +3674,7 @@ __global__ void k_cap_check(uint64_t cap, uint32_t* __restrict__ offsets, int B,
 // waves), finds those with a record by ballot and copies them one after another, lanes over
 // bytes; wavefronts stride over the batch. Most anchors have no record: a workgroup per anchor
 // spent 212 us on 1.0M anchors with 130,000 records, where this takes about 20, and a wave per
-// candidate entry 700 us on 10.0M entries with 707,000 records, about 170. Returns the wave's
+// candidate entry 700 us on 10.0M entries with 707,000 records, about 150. Returns the wave's
 // records.
 constexpr int kGatherGrid = 4096;
 constexpr uint64_t kGatherSmall = uint64_t(kGatherGrid) * (kBlock / kWave) * kWave / 8;
