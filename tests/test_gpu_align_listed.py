@@ -14,8 +14,8 @@ def tandem(lmin, lmax, genome_length, seed=51):
     return reads.storage_from_sim(s, use_qualities=False)
 
 
-def context(rs, variant):
-    eng = engine.CareEngine(0, kmerlength=20, align_variant=variant)
+def context(rs, variant, **opts):
+    eng = engine.CareEngine(0, kmerlength=20, align_variant=variant, **opts)
     eng.set_reads(rs)
     eng.build_tables()
     return eng
@@ -30,6 +30,22 @@ def test_small_batches_of_listed_anchors(lengths):
         assert m.correct(first, n) == w.correct(first, n)
     m.close()
     w.close()
+
+
+@pytest.mark.parametrize("opts", [dict(use_graphs=1), dict(use_graphs=1, batch_size=500), dict(batch_size=500),
+                                  dict(batch_size=500, pipeline_capacity=4), dict(sync_batches=1), dict(correct_candidates=1)],
+                         ids=lambda o: "-".join(f"{k}={v}" for k, v in o.items()))
+def test_listed_anchors_on_every_schedule(opts):
+    # repeated passes: the lists are emptied before each batch, in captured batches too
+    rs = tandem(150, 150, genome_length=12_000, seed=52)
+    print(f"[{opts}] reads={rs.n}", flush=True)
+    w = context(rs, 1, correct_candidates=opts.get("correct_candidates", 0))
+    want = w.correct()
+    w.close()
+    m = context(rs, 0, **opts)
+    for _ in range(4):
+        assert m.correct() == want
+    m.close()
 
 
 def test_long_reads_of_low_complexity_cost_what_the_scan_costs():
